@@ -27,8 +27,8 @@
 // the five coefficient arrays.
 //
 // The member functions of Plan<T> are defined by topic in plan_setup.cpp,
-// plan_shots.cpp, plan_step.cpp, plan_forward.cpp, plan_adjoint.cpp,
-// plan_discrete.cpp and plan_results.cpp; each file instantiates its own for
+// plan_shots.cpp, plan_step.cpp, plan_resident.cpp, plan_forward.cpp,
+// plan_adjoint.cpp, plan_discrete.cpp and plan_results.cpp; each file instantiates its own for
 // the four arithmetic types (PSV_FOR_EACH_PRECISION).
 #pragma once
 
@@ -43,6 +43,7 @@
 
 #include "psv_aux.h"
 #include "psv_discrete.h"
+#include "psv_resident.h"
 #include "psv_step.h"
 #include "psvfwi.h"
 
@@ -171,6 +172,8 @@ template <typename T>
 class Plan final : public psvfwi_plan {
 public:
     static constexpr int kDefaultTz = 8;
+    // fewest steps a resident launch is worth: it loads the whole state and writes it back
+    static constexpr int kResidentMin = 8;
 
     // ---------------------------------------------------------- plan_setup.cpp
     explicit Plan(const psvfwi_grid_desc& g);
@@ -233,6 +236,27 @@ private:
         // per-tile lists for the tile height they were built for
         DBuf<int> tinj_off, tinj_idx, trec_off, trec_idx;
         int built_tz = -1;
+        // host copies of inj_grp, inj_row and rec_zxc, and the resident loop's point tables for
+        // the tiles they were built for
+        std::vector<int> grp_h, row_h, zxc_h;
+        DBuf<int> res_off, res_head, res_id;
+        int res_gen = -1;
+    };
+
+    // the resident time loop (plan_resident.cpp): the tiles chosen for a batch of `slots`
+    // shots (shape < 0: it does not fit), conc slots per launch
+    struct Resident {
+        int slots = 0, shape = -1, conc = 0, waves = 0, rows = 0, rows_edge = 0, gen = 0;
+        bool failed = false;    // refused or aborted once: the plan keeps to the split step
+        bool uploaded = false;
+        int kdiv = 0;           // some CPML K differs from 1
+        std::vector<psv::ResTile> h;
+        DBuf<psv::ResTile> tiles;
+        DBuf<unsigned long long> exch;
+        size_t exch_slot = 0;
+        int xpitch = 0;
+        unsigned tag = 1;
+        int* aborted = nullptr;  // pinned host memory the kernel writes when a wait runs out
     };
 
     // device pointers into one saved state (state_copy layout)
@@ -268,6 +292,15 @@ private:
     psvfwi_status collect_samples();
     psvfwi_status capture_steps(psv::StepParams<T> p0, int mode, int dir, State<T>& st, State<T>& alt,
                                 const Tables& tab, bool fwd_sig, hipGraphExec_t* out);
+
+    // ------------------------------------------------------- plan_resident.cpp
+    std::vector<psv::ResTile> resident_tiles(const psv::ResShape& sh) const;
+    bool resident_ready();
+    psvfwi_status resident_points(Tables& t);
+    psvfwi_status resident_prepare();
+    psvfwi_status launch_resident(State<T>& st, Tables& tab, bool fwd_sig, int mode, int kind, int it0, int it1,
+                                  int flags, int tf0, bool one_plane = false);
+    bool resident_failed();
 
     // -------------------------------------------------------- plan_adjoint.cpp
     psvfwi_status adjoint_step(int it, int flags, int tf0);
@@ -312,10 +345,12 @@ private:
     // batch as one group.
     int group_size() const { return (lg_ > 0 && !fused()) ? std::min(lg_, nslots_) : nslots_; }
 
-    void set_group(int w0)
+    void set_group(int w0) { set_group(w0, group_size()); }
+
+    void set_group(int w0, int size)
     {
         w0_ = w0;
-        w1_ = std::min(nslots_, w0 + group_size());
+        w1_ = std::min(nslots_, w0 + size);
     }
 
     void all_slots()
@@ -404,6 +439,8 @@ private:
     int fpad_ = 1, ppad_ = 0, tp_ = 2, pitch_ = 0, rows_ = 0, org_ = 0, pnx_ = 0, pnz_ = 0, tz_ = 16;
     size_t fst_ = 0, xst_ = 0, zst_ = 0;
     bool parity_ = false;
+    bool tile_auto_ = true;  // no tile height chosen by the caller: the resident loop where it fits
+    Resident res_;
     int graph_steps_ = 0;  // > 0: time loops replay captured chunks of this many steps
     int band_ = 0;         // block order of a batch (StepParams::band)
     int lg_ = 0;           // shots per launch group (0: the whole batch)
@@ -477,6 +514,7 @@ private:
     float tune_ms_[kNumCand] = {};
     hipEvent_t sample_ev_[kMaxSamples][3] = {};
     int samp_kind_[kMaxSamples] = {};
+    int samp_steps_[kMaxSamples] = {};  // time steps the sample covers
     int nsamp_ = 0;
     double kus_[3][2] = {};
     int kn_[3] = {};

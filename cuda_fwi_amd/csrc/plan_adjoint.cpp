@@ -66,6 +66,9 @@ psvfwi_status Plan<T>::adjoint(int flags)
     const bool ckpt = grad && store_mode_ == PSVFWI_STORE_CHECKPOINT;
     if (grad && !ckpt && !store_loaded_) return fail(PSVFWI_E_STATE, "adjoint: forward store missing");
 
+    const bool resident = !(ckpt && ck_used_k_ < kResidentMin) && resident_ready();
+    if (resident) PSV_TRY(resident_prepare());
+    const int gsize = resident ? res_.conc : group_size();
     PSV_TRY(alloc_state(main_));
     PSV_TRY(zero_state(main_));
     if (fused()) {
@@ -84,7 +87,7 @@ psvfwi_status Plan<T>::adjoint(int flags)
         PSV_HIP(psv::launch_fill<T>(grad_.p, grad_.n, (T)0, stream_));
     }
     const int aflags = (energy ? psv::kEnergy : 0) | (grad ? psv::kStore : 0);
-    PSV_TRY(ensure_all_tile_lists());
+    if (!resident) PSV_TRY(ensure_all_tile_lists());
 
     PSV_TRY(begin_samples());
     PSV_HIP(hipEventRecord(ev0_, stream_));
@@ -99,9 +102,13 @@ psvfwi_status Plan<T>::adjoint(int flags)
         }
         PSV_TRY(alloc_store((ck_used_k_ + w_.dt - 1) / w_.dt + 1));
     }
-    for (int w0 = 0; w0 < nslots_; w0 += group_size()) {
-        set_group(w0);
+    for (int w0 = 0; w0 < nslots_; w0 += gsize) {
+        set_group(w0, gsize);
         const int ntg = group_nt();
+        if (resident && !ckpt) {
+            PSV_TRY(launch_resident(main_, adj_tab_, false, psv::kAdjoint, 1, 0, ntg, aflags, 0));
+            continue;
+        }
         if (!ckpt) {
             for (int it = ntg - 1; it >= 0; it--) {
                 if (graph_steps_ > 0) {
@@ -135,6 +142,11 @@ psvfwi_status Plan<T>::adjoint(int flags)
             const int tf0 = (t0 + w_.dt - 1) / w_.dt;
             // replay the segment forward from its checkpoint into the segment store
             PSV_TRY(restore_checkpoint(c, active(t0)));
+            if (resident) {
+                PSV_TRY(launch_resident(replay_, fwd_tab_noreceivers_, true, psv::kForward, 2, t0, t1, psv::kStore, tf0));
+                PSV_TRY(launch_resident(main_, adj_tab_, false, psv::kAdjoint, 1, t0, t1, aflags, tf0));
+                continue;
+            }
             for (int it = t0; it < t1; it++) {
                 psv::StepParams<T> p = base_params(replay_, fwd_tab_noreceivers_, true);
                 p.it = it;
@@ -151,6 +163,7 @@ psvfwi_status Plan<T>::adjoint(int flags)
     PSV_HIP(hipEventRecord(ev1_, stream_));
     PSV_HIP(hipStreamSynchronize(stream_));
     for (hipGraphExec_t ex : graphs) PSV_HIP(hipGraphExecDestroy(ex));
+    if (resident && resident_failed()) return adjoint(flags);
     float ms = 0;
     PSV_HIP(hipEventElapsedTime(&ms, ev0_, ev1_));
     last_ms_ = ms;

@@ -36,19 +36,32 @@ psvfwi_status Plan<T>::forward(int flags)
     if (full) PSV_TRY(alloc_store(1 + (ntmax_ - 1) / w_.dt));
     if (ckpt) PSV_TRY(alloc_checkpoints(every ? 0 : kint));
     const bool snap = snap_interval_ > 0;
+    // short checkpoint intervals and snapshots need the state in memory after every few steps
+    const bool resident = !snap && !every && !(ckpt && kint < kResidentMin) && resident_ready();
+    if (resident) PSV_TRY(resident_prepare());
+    const int gsize = resident ? res_.conc : group_size();
     if (snap) PSV_HIP(snaps_.alloc((size_t)((ntmax_ - 1) / snap_interval_ + 1) * nslots_ * fst_));
     snaps_taken_ = snap;
 
-    PSV_TRY(ensure_all_tile_lists());
+    // (the discrete adjoint replays with the split step)
+    if (!resident || discrete) PSV_TRY(ensure_all_tile_lists());
     PSV_TRY(begin_samples());
     PSV_HIP(hipEventRecord(ev0_, stream_));
     launches_ = 0;
     const int fflags = (energy ? psv::kEnergy : 0) | (full ? psv::kStore : 0);
     std::vector<hipGraphExec_t> graphs;
     AllSlotsAfter restore{this};
-    for (int w0 = 0; w0 < nslots_; w0 += group_size()) {
-        set_group(w0);
+    for (int w0 = 0; w0 < nslots_; w0 += gsize) {
+        set_group(w0, gsize);
         const int ntg = group_nt();
+        if (resident) {
+            const int chunk = ckpt ? kint : ntg;
+            for (int it = 0; it < ntg; it += chunk) {
+                if (ckpt) PSV_TRY(save_checkpoint(it / kint, active(it)));
+                PSV_TRY(launch_resident(main_, fwd_tab_, true, psv::kForward, 0, it, std::min(it + chunk, ntg), fflags, 0));
+            }
+            continue;
+        }
         for (int it = 0; it < ntg; it++) {
             const int na = active(it);
             if (graph_steps_ > 0 && !snap && !ckpt) {
@@ -94,6 +107,7 @@ psvfwi_status Plan<T>::forward(int flags)
     PSV_HIP(hipEventRecord(ev1_, stream_));
     PSV_HIP(hipStreamSynchronize(stream_));
     for (hipGraphExec_t ex : graphs) PSV_HIP(hipGraphExecDestroy(ex));
+    if (resident && resident_failed()) return forward(flags);
     float ms = 0;
     PSV_HIP(hipEventElapsedTime(&ms, ev0_, ev1_));
     last_ms_ = ms;

@@ -1,0 +1,284 @@
+// plan_resident.cpp -- the resident time loop of a plan (psv_resident.inc): when it is
+// used, the partition of the grid into tiles, the point tables and the launch.
+#include <cstdio>
+
+#include "plan.h"
+
+namespace psvplan {
+
+namespace {
+
+// The rows of one column of tiles.  A tile is interior when every stress cell it computes
+// (2 cells around the owned ones) is updated, outside the CPML strips and below the
+// free-surface row: rows in [zlo, zhi) (and xin, the same in x).  Interior tiles take up to
+// `own` rows, edge tiles up to `own_edge`; the fewest tiles that cover the column.
+void tile_column(int nzt, int zlo, int zhi, bool xin, int own, int own_edge, int x0, int x1, int xr,
+                 std::vector<psv::ResTile>& out)
+{
+    // need[z]: tiles for the rows from z on; step[z]: height of the first, negative for interior
+    std::vector<int> need((size_t)nzt + 1, 0), step((size_t)nzt + 1, 0);
+    for (int z = nzt - 1; z >= 0; z--) {
+        const int he = std::min(own_edge, nzt - z);
+        need[(size_t)z] = 1 + need[(size_t)(z + he)];
+        step[(size_t)z] = he;
+        const int hi = std::min(own, zhi - 2 - z);
+        if (xin && z - 2 >= zlo && hi > 0 && 1 + need[(size_t)(z + hi)] <= need[(size_t)z]) {
+            need[(size_t)z] = 1 + need[(size_t)(z + hi)];
+            step[(size_t)z] = -hi;
+        }
+    }
+    for (int z = 0; z < nzt;) {
+        const int h = step[(size_t)z] < 0 ? -step[(size_t)z] : step[(size_t)z];
+        psv::ResTile t{};
+        t.z0 = z;
+        t.z1 = z + h;
+        t.x0 = x0;
+        t.x1 = x1;
+        t.zr = std::max(0, z - psv::kResHalo);
+        t.xr = xr;
+        t.edge = step[(size_t)z] < 0 ? 0 : 1;
+        out.push_back(t);
+        z += h;
+    }
+}
+
+}  // namespace
+
+// The tiles of the grid for a shape.
+template <typename T>
+std::vector<psv::ResTile> Plan<T>::resident_tiles(const psv::ResShape& sh) const
+{
+    const int nzt = g_.nzt, nxt = g_.nxt, H = fpad_;
+    const bool pml = g_.npml > 0;
+    const int zlo = g_.fsurf ? H + 1 : (pml ? ppad_ + 1 : H);
+    const int zhi = pml ? nzt - ppad_ - 1 : nzt - H;
+    const int xlo = pml ? ppad_ + 1 : H, xhi = pml ? nxt - ppad_ - 1 : nxt - H;
+    const int own = sh.rows * sh.waves - 2 * psv::kResHalo;
+    const int own_edge = sh.rows_edge * sh.waves - 2 * psv::kResHalo;
+    std::vector<psv::ResTile> out;
+    // columns: the first and last tile have a halo on one side only
+    const int W = psv::kResOwnX, end = W + psv::kResHalo;
+    const int ncol = nxt <= 64 ? 1 : (nxt <= 2 * end ? 2 : 2 + (nxt - 2 * end + W - 1) / W);
+    for (int c = 0, x = 0; c < ncol; c++) {
+        // even widths, within what each column can hold
+        const int left = ncol - 1 - c, rest = left == 0 ? 0 : (left - 1) * W + end;
+        const int most = ncol == 1 ? 64 : (c == 0 || left == 0 ? end : W);
+        const int x1 = x + std::min(most, std::max((nxt - x + left) / (left + 1), nxt - x - rest));
+        const bool xin = x - 2 >= xlo && x1 + 2 <= xhi;
+        tile_column(nzt, zlo, zhi, xin, own, own_edge, x, x1, std::max(0, x - psv::kResHalo), out);
+        x = x1;
+    }
+    return out;
+}
+
+// Whether the plan's runs can take the resident loop, and its shape for the current batch.
+// Not for a caller who chose a tile height; not for CPML profiles that couple the strips
+// (the reference's arrays give the innermost cells of the two strips of an axis one memory
+// cell, which stays zero only while a = a_half = 0 there), nor for grids whose strips meet.
+template <typename T>
+bool Plan<T>::resident_ready()
+{
+    const psv::ResShape* shapes = nullptr;
+    const int n = psv::resident_shapes<T>(&shapes);
+    if (n == 0 || !tile_auto_ || res_.failed || nslots_ < 1) return false;
+    if (g_.npml > 0) {
+        if (!have_pml_ || h_pml_[(size_t)g_.npml] != 0.0 || h_pml_[(size_t)3 * tp_ + g_.npml] != 0.0) return false;
+        if (g_.nxt - 2 * ppad_ < 3 || g_.nzt - 2 * ppad_ < 3) return false;
+    }
+    // every tile needs room for the mirror rows and the rim of a neighbour
+    if (g_.nxt < 16 || g_.nzt < 16) return false;
+    if (res_.slots == nslots_) return res_.shape >= 0;
+    res_.slots = nslots_;
+    res_.shape = -1;
+    double best = 0;
+    for (int i = 0; i < n; i++) {
+        const std::vector<psv::ResTile> t = resident_tiles(shapes[i]);
+        int cap = 1 << 30;
+        for (int mode : {(int)psv::kForward, (int)psv::kAdjoint}) {
+            int c = 0;
+            if (psv::resident_capacity<T>(g_.fdorder, mode, i, &c) != hipSuccess) c = 0;
+            cap = std::min(cap, c);
+        }
+        if ((int)t.size() > cap) continue;
+        const int conc = std::min(nslots_, cap / (int)t.size());
+        const int rounds = (nslots_ + conc - 1) / conc;
+        const double cost = rounds * (3.0 + 0.35 * shapes[i].rows);
+        if (res_.shape < 0 || cost < best) {
+            best = cost;
+            res_.shape = i;
+            res_.conc = conc;
+            res_.h = t;
+        }
+    }
+    if (res_.shape < 0) return false;
+    res_.waves = shapes[res_.shape].waves;
+    res_.rows = shapes[res_.shape].rows;
+    res_.rows_edge = shapes[res_.shape].rows_edge;
+    res_.gen++;
+    res_.uploaded = false;
+    return true;
+}
+
+// the point tables of a Tables object for the current tiles (ResPoints)
+template <typename T>
+psvfwi_status Plan<T>::resident_points(Tables& t)
+{
+    if (t.res_gen == res_.gen) return PSVFWI_OK;
+    const int ntile = (int)res_.h.size();
+    const int nw = res_.waves;
+    struct Layer {
+        int head;
+        std::vector<int> id;
+    };
+    std::vector<std::vector<Layer>> lay((size_t)nslots_ * ntile * nw);
+    // entry `v` of component `comp` at (z, x): the first layer of its wave, row and component
+    // whose lane is free, so that entries of one cell keep their order
+    auto add = [&](int slot, int k, int z, int x, int comp, int rec, int v) {
+        const psv::ResTile& q = res_.h[(size_t)k];
+        const int R = q.edge ? res_.rows_edge : res_.rows;
+        const int row = z - q.zr, lane = x - q.xr;
+        std::vector<Layer>& l = lay[((size_t)slot * ntile + k) * nw + (size_t)(row / R)];
+        const int head = (row % R) | comp << 8 | rec << 16;
+        for (Layer& y : l)
+            if (y.head == head && y.id[(size_t)lane] < 0) {
+                y.id[(size_t)lane] = v;
+                return;
+            }
+        l.push_back(Layer{head, std::vector<int>(64, -1)});
+        l.back().id[(size_t)lane] = v;
+    };
+    for (int s = 0; s < nslots_; s++)
+        for (int rec = 0; rec < 2; rec++) {
+            const std::vector<int>& off = rec ? t.rec_off : t.grp_off;
+            for (int g = off[(size_t)s]; g < off[(size_t)s + 1]; g++) {
+                const int* e = rec ? &t.zxc_h[3 * (size_t)g] : &t.grp_h[5 * (size_t)g];
+                const int z = e[0], x = e[1], comp = e[2];
+                for (int k = 0; k < ntile; k++) {
+                    const psv::ResTile& q = res_.h[(size_t)k];
+                    // stress sources act on the stresses a tile computes around its own cells too
+                    const int ring = !rec && comp == 4 ? 2 : 0;
+                    if (z < q.z0 - ring || z >= q.z1 + ring || x < q.x0 - ring || x >= q.x1 + ring) continue;
+                    if (rec) add(s, k, z, x, comp, 1, g - off[(size_t)s]);
+                    else
+                        for (int j = 0; j < e[4]; j++) add(s, k, z, x, comp, 0, t.row_h[(size_t)(e[3] + j)]);
+                }
+            }
+        }
+    std::vector<int> off(lay.size() + 1, 0), head, id;
+    for (size_t i = 0; i < lay.size(); i++) {
+        off[i + 1] = off[i] + (int)lay[i].size();
+        for (const Layer& y : lay[i]) {
+            head.push_back(y.head);
+            id.insert(id.end(), y.id.begin(), y.id.end());
+        }
+    }
+    PSV_HIP(t.res_off.alloc(off.size()));
+    PSV_HIP(t.res_head.alloc(std::max<size_t>(head.size(), 1)));
+    PSV_HIP(t.res_id.alloc(std::max<size_t>(id.size(), 64)));
+    PSV_HIP(hipMemcpy(t.res_off.p, off.data(), off.size() * sizeof(int), hipMemcpyHostToDevice));
+    if (!head.empty()) {
+        PSV_HIP(hipMemcpy(t.res_head.p, head.data(), head.size() * sizeof(int), hipMemcpyHostToDevice));
+        PSV_HIP(hipMemcpy(t.res_id.p, id.data(), id.size() * sizeof(int), hipMemcpyHostToDevice));
+    }
+    t.res_gen = res_.gen;
+    return PSVFWI_OK;
+}
+
+// tiles, exchange buffer and flag of the resident loop
+template <typename T>
+psvfwi_status Plan<T>::resident_prepare()
+{
+    if (!res_.uploaded) {
+        PSV_HIP(res_.tiles.alloc(res_.h.size()));
+        PSV_HIP(hipMemcpy(res_.tiles.p, res_.h.data(), res_.h.size() * sizeof(psv::ResTile), hipMemcpyHostToDevice));
+        res_.uploaded = true;
+    }
+    res_.xpitch = (int)round_up((size_t)g_.nxt, 8);
+    res_.exch_slot = (size_t)2 * g_.nzt * res_.xpitch * (2 * sizeof(T) / 4);
+    const size_t need = res_.exch_slot * (size_t)res_.conc;
+    if (!res_.exch.p || res_.exch.cap < need) {
+        PSV_HIP(res_.exch.alloc(need));
+        PSV_HIP(psv::launch_fill<unsigned long long>(res_.exch.p, res_.exch.cap, 0ull, stream_));
+        res_.tag = 1;
+    }
+    if (!res_.aborted) {
+        PSV_HIP(hipHostMalloc(reinterpret_cast<void**>(&res_.aborted), sizeof(int), hipHostMallocMapped));
+        *res_.aborted = 0;
+    }
+    return PSVFWI_OK;
+}
+
+// Steps [it0, it1) of the current launch group in one launch: forward in time, or for the
+// adjoint backward from each shot's min(it1, nt) - 1.
+template <typename T>
+psvfwi_status Plan<T>::launch_resident(State<T>& st, Tables& tab, bool fwd_sig, int mode, int kind, int it0, int it1,
+                                       int flags, int tf0, bool one_plane)
+{
+    PSV_TRY(resident_points(tab));
+    const int steps = it1 - it0;
+    if (res_.tag > 0xffffffffu - (unsigned)steps - 2u) {
+        PSV_HIP(psv::launch_fill<unsigned long long>(res_.exch.p, res_.exch.cap, 0ull, stream_));
+        res_.tag = 1;
+    }
+    psv::ResidentParams<T> a{};
+    a.p = base_params(st, tab, fwd_sig);
+    a.p.nslots = active(it0);
+    a.p.flags = flags;
+    a.p.tf0 = tf0;
+    a.tiles = res_.tiles.p;
+    a.ntile = (int)res_.h.size();
+    a.it0 = it0;
+    a.it1 = it1;
+    const size_t per = (size_t)a.ntile * res_.waves;
+    a.pts.off = tab.res_off.p + (size_t)w0_ * per;
+    a.pts.head = tab.res_head.p;
+    a.pts.id = tab.res_id.p;
+    a.tf_stride = one_plane ? 0 : (size_t)5 * nfz_ * nfx_;
+    a.exch = res_.exch.p;
+    a.exch_slot = res_.exch_slot;
+    a.xpitch = res_.xpitch;
+    a.tag = res_.tag;
+    a.aborted = res_.aborted;
+    a.kdiv = res_.kdiv;
+    res_.tag += (unsigned)steps;
+    const bool sample = kind >= 0 && sample_ev_[0][0] && nsamp_ < kMaxSamples;
+    if (sample) PSV_HIP(hipEventRecord(sample_ev_[nsamp_][0], stream_));
+    const hipError_t e = psv::launch_resident<T>(a, g_.fdorder, mode, res_.shape, stream_);
+    if (e != hipSuccess) {
+        // refused (no cooperative launch here): the caller runs the split step instead
+        (void)hipGetLastError();
+        *res_.aborted = 1;
+        return PSVFWI_OK;
+    }
+    if (sample) {
+        PSV_HIP(hipEventRecord(sample_ev_[nsamp_][1], stream_));
+        PSV_HIP(hipEventRecord(sample_ev_[nsamp_][2], stream_));
+        samp_kind_[nsamp_] = kind;
+        samp_steps_[nsamp_] = steps;
+        nsamp_++;
+    }
+    if (kind >= 0) launches_ += steps;
+    return PSVFWI_OK;
+}
+
+// After the stream has drained: a resident run whose waits ran out, or that was refused,
+// has left the state unusable; the plan then keeps to the split step and the run starts over.
+template <typename T>
+bool Plan<T>::resident_failed()
+{
+    if (!res_.aborted || *res_.aborted == 0) return false;
+    *res_.aborted = 0;
+    res_.failed = true;
+    return true;
+}
+
+#define PSV_INSTANTIATE(T) \
+    template std::vector<psv::ResTile> Plan<T>::resident_tiles(const psv::ResShape&) const; \
+    template bool Plan<T>::resident_ready(); \
+    template psvfwi_status Plan<T>::resident_points(Tables&); \
+    template psvfwi_status Plan<T>::resident_prepare(); \
+    template psvfwi_status Plan<T>::launch_resident(State<T>&, Tables&, bool, int, int, int, int, int, int, bool); \
+    template bool Plan<T>::resident_failed();
+PSV_FOR_EACH_PRECISION(PSV_INSTANTIATE)
+
+}  // namespace psvplan

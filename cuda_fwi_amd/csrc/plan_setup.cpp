@@ -40,6 +40,7 @@ Plan<T>::~Plan()
     if (side_.join) (void)hipEventDestroy(side_.join);
     if (side_.stream) (void)hipStreamDestroy(side_.stream);
     if (stream_) (void)hipStreamDestroy(stream_);
+    if (res_.aborted) (void)hipHostFree(res_.aborted);
 }
 
 template <typename T>
@@ -66,6 +67,9 @@ psvfwi_status Plan<T>::set_pml(const double* prof)
     std::vector<T> h((size_t)6 * tp_);
     for (size_t i = 0; i < h.size(); i++) h[i] = (T)prof[i];
     h_pml_.assign(prof, prof + h.size());
+    res_.kdiv = 0;
+    for (int i = 0; i < tp_; i++)
+        if (prof[(size_t)2 * tp_ + i] != 1.0 || prof[(size_t)5 * tp_ + i] != 1.0) res_.kdiv = 1;
     PSV_HIP(hipMemcpyAsync(pml_.p, h.data(), h.size() * sizeof(T), hipMemcpyHostToDevice, stream_));
     PSV_HIP(hipStreamSynchronize(stream_));
     have_pml_ = true;
@@ -158,11 +162,13 @@ psvfwi_status Plan<T>::set_snapshots(int interval, int field)
 template <typename T>
 psvfwi_status Plan<T>::set_tile(int tz)
 {
-    if (tz == 0) tz = kDefaultTz;
+    const bool chosen = tz != 0;
+    if (!chosen) tz = kDefaultTz;
     if (!tile_ok(tz))
         return fail(PSVFWI_E_ARG, "set_tile: tile height must be 4, 8, 16 or (FP32) 32 (split step), -8 or -16 (fused step), "
                                   "-32 or -64 (z-marching step)");
     tz_ = tz;
+    tile_auto_ = !chosen;
     return PSVFWI_OK;
 }
 

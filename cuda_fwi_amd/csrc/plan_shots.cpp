@@ -95,6 +95,9 @@ psvfwi_status Plan<T>::build_injection(Tables& t, bool adjoint_sources, bool wit
     if (with_signals) fwd_sig_h_ = sig;
     // inj_row holds signal rows relative to the shot; the kernel adds sig_off[slot]
     t.grp_off = off;
+    t.grp_h = grp;
+    t.row_h = row;
+    t.res_gen = -1;
     t.grp_zx.clear();
     if (with_signals) fwd_grp_comp_.clear();
     for (size_t q = 0; q < grp.size(); q += 5) {
@@ -134,6 +137,8 @@ psvfwi_status Plan<T>::build_receivers(Tables& t, bool none)
         off.push_back((int)(zxc.size() / 3));
     }
     t.rec_off = off;
+    t.zxc_h = zxc;
+    t.res_gen = -1;
     t.built_tz = -1;
     PSV_HIP(t.rec_first.alloc(off.size()));
     PSV_HIP(t.rec_zxc.alloc(std::max<size_t>(zxc.size(), 1)));

@@ -65,6 +65,31 @@ psvfwi_status Plan<T>::autotune(int steps, int* best)
     const int cand[kNumCand] = {4, 8, 16, 32, -8, -16, -32, -64};
     float best_ms = 1e30f;
     int best_tz = tz_;
+    // the resident loop first, where it fits
+    float res_ms = 1e30f;
+    tile_auto_ = true;
+    if (resident_ready()) {
+        tz_ = kDefaultTz;
+        PSV_TRY(resident_prepare());
+        AllSlotsAfter restore{this};
+        for (int rep = 0; rep < 2; rep++) {
+            PSV_TRY(zero_state(main_));
+            PSV_HIP(hipEventRecord(ev0_, stream_));
+            for (int w0 = 0; w0 < nslots_; w0 += res_.conc) {
+                set_group(w0, res_.conc);
+                const int nstep = std::min(steps, group_nt());
+                PSV_TRY(launch_resident(main_, fwd_tab_noreceivers_, true, psv::kForward, -1, 0, nstep, 0, 0));
+                if (adj)
+                    PSV_TRY(launch_resident(main_, adj_tab_, false, psv::kAdjoint, -1, 0, nstep, psv::kStore, 0, true));
+            }
+            all_slots();
+            PSV_HIP(hipEventRecord(ev1_, stream_));
+            PSV_HIP(hipStreamSynchronize(stream_));
+            PSV_HIP(hipEventElapsedTime(&res_ms, ev0_, ev1_));
+        }
+        if (resident_failed()) res_ms = 1e30f;
+    }
+    tile_auto_ = false;
     for (int c = 0; c < kNumCand; c++) {
         tune_ms_[c] = -1;
         if (!tile_ok(cand[c])) continue;
@@ -116,7 +141,11 @@ psvfwi_status Plan<T>::autotune(int steps, int* best)
             lg_ = best_lg;
         }
     }
-    if (best) *best = best_tz;
+    // the resident loop stays the plan's choice (as set_tile(0) makes it) where it was the
+    // fastest; the value returned is the split or fused step's either way
+    tile_auto_ = res_ms < best_ms;
+    if (tile_auto_) tz_ = kDefaultTz;
+    if (best) *best = tile_auto_ ? kDefaultTz : best_tz;
     // the candidates ran in the plan's own state, store and gradient buffers
     drop_results();
     return PSVFWI_OK;
@@ -198,6 +227,7 @@ psvfwi_status Plan<T>::launch_timed(const psv::StepParams<T>& p, int mode, int k
         PSV_TRY(launch_plain(p, mode, st, alt, sample_ev_[nsamp_][1]));
         PSV_HIP(hipEventRecord(sample_ev_[nsamp_][2], stream_));
         samp_kind_[nsamp_] = kind;
+        samp_steps_[nsamp_] = 1;
         nsamp_++;
     } else {
         PSV_TRY(launch_plain(p, mode, st, alt));
@@ -228,8 +258,8 @@ psvfwi_status Plan<T>::collect_samples()
             float m1 = 0, m2 = 0;
             PSV_HIP(hipEventElapsedTime(&m1, sample_ev_[i][0], sample_ev_[i][1]));
             PSV_HIP(hipEventElapsedTime(&m2, sample_ev_[i][1], sample_ev_[i][2]));
-            a += m1;
-            b += m2;
+            a += m1 / samp_steps_[i];
+            b += m2 / samp_steps_[i];
             n++;
         }
         kus_[k][0] = n ? a / n * 1e3 : 0;

@@ -166,6 +166,7 @@ template hipError_t launch_grad_sum<double>(const double*, size_t, const int*, i
 template hipError_t launch_fill<float>(float*, size_t, float, hipStream_t);
 template hipError_t launch_fill<double>(double*, size_t, double, hipStream_t);
 template hipError_t launch_fill<int>(int*, size_t, int, hipStream_t);
+template hipError_t launch_fill<unsigned long long>(unsigned long long*, size_t, unsigned long long, hipStream_t);
 template hipError_t launch_misfit<dfloat>(const dfloat*, const double*, dfloat*, const size_t*,
                                           const size_t*, int, int, double, double*, double*, int*,
                                           hipStream_t);

@@ -1,0 +1,70 @@
+// psv_resident.h -- launch parameters of the resident time loop: many steps of a
+// shot in one cooperative launch, its wavefields held in registers.
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stddef.h>
+
+#include "psv_step.h"
+
+namespace psv {
+
+constexpr int kResHalo = 4;                    // velocity halo of a tile: two half-steps of two cells
+constexpr int kResOwnX = 64 - 2 * kResHalo;    // columns a tile owns between two others
+
+// One workgroup's tile: it owns the cells [z0, z1) x [x0, x1) and holds the region
+// that starts at (zr, xr): kResHalo more cells on every side that has a neighbour.
+struct ResTile {
+    int z0, z1, x0, x1;
+    int zr, xr;
+    int edge;  // the region meets a CPML strip, the free surface or the grid's frame
+    int pad;
+};
+
+// Point sources and receivers of a (slot, tile, wave): layers of at most one entry per
+// lane, in the order they act; head: row | comp << 8 | receiver << 16; id: signal row or
+// receiver of the lane (-1: none).
+struct ResPoints {
+    const int* off;   // [(slot * ntile + tile) * waves + wave] into head
+    const int* head;
+    const int* id;    // [layer][64]
+};
+
+template <typename T>
+struct ResidentParams {
+    StepParams<T> p;         // fields, model and tables of the launch's first slot
+    const ResTile* tiles;
+    int ntile;
+    int it0, it1;            // steps [it0, it1), each slot up to its own nt
+    ResPoints pts;
+    size_t tf_stride;        // elements from one stored time to the next
+    // velocity exchange: per slot two generations of [nzt][xpitch] cells, each value a
+    // 64-bit word {tag, 32 bits of the value}
+    unsigned long long* exch;
+    size_t exch_slot;        // words per slot
+    int xpitch;
+    unsigned tag;            // tag of the launch's first step
+    int* aborted;            // host memory: set when a wait ran out
+    int kdiv;                // some CPML K differs from 1
+};
+
+// Tile shapes a launch can take: waves of a workgroup, stacked in z, and rows per wave of
+// the interior and of the edge tiles.
+struct ResShape {
+    int waves, rows, rows_edge;
+};
+
+// The shapes built for a type (sizeof(T) bytes per value), smallest first; returns their
+// number (0: the type has no resident loop).
+template <typename T>
+int resident_shapes(const ResShape** out);
+
+// Workgroups of one launch that are resident together on the current device.
+template <typename T>
+hipError_t resident_capacity(int order, int mode, int shape, int* workgroups);
+
+// nslots * ntile workgroups; hipErrorInvalidValue for an order, mode or shape not built.
+template <typename T>
+hipError_t launch_resident(const ResidentParams<T>& a, int order, int mode, int shape, hipStream_t s);
+
+}  // namespace psv
