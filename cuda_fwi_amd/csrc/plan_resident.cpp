@@ -1,6 +1,6 @@
 // plan_resident.cpp -- the resident time loop of a plan (psv_resident.inc): when it is
 // used, the partition of the grid into tiles, the point tables and the launch.
-#include <cstdio>
+#include <type_traits>
 
 #include "plan.h"
 
@@ -71,6 +71,16 @@ std::vector<psv::ResTile> Plan<T>::resident_tiles(const psv::ResShape& sh) const
     return out;
 }
 
+// A split step of `n` shots in us: two launches that a small grid does not fill, then the
+// bytes it moves.  Fitted to one MI355X (order 4, forward and adjoint mean): FP32 12.7 on
+// 55 k cells, 17.3 on 0.63 M, 25 on 1.08 M and 25 on 16 x 52 k; FP64 15 on 0.2 M, 28 on
+// 0.63 M, 38 on 0.82 M; compensated FP32 20 on 55 k and 21 on 0.2 M.
+static double split_step_us(double cells, int esize, bool dwords)
+{
+    const double floor = dwords ? 20.0 : 12.5;
+    return std::max(floor, 5.0 + cells * (esize == 4 ? 19e-6 : 39e-6));
+}
+
 // Whether the plan's runs can take the resident loop, and its shape for the current batch.
 // Not for a caller who chose a tile height; not for CPML profiles that couple the strips
 // (the reference's arrays give the innermost cells of the two strips of an axis one memory
@@ -90,7 +100,8 @@ bool Plan<T>::resident_ready()
     if (res_.slots == nslots_) return res_.shape >= 0;
     res_.slots = nslots_;
     res_.shape = -1;
-    double best = 0;
+    // the shots run conc at a time, rounds times over; the split step takes them together
+    double best = split_step_us((double)nslots_ * g_.nzt * g_.nxt, (int)sizeof(T), std::is_same<T, psv::dfloat>::value);
     for (int i = 0; i < n; i++) {
         const std::vector<psv::ResTile> t = resident_tiles(shapes[i]);
         int cap = 1 << 30;
@@ -102,8 +113,8 @@ bool Plan<T>::resident_ready()
         if ((int)t.size() > cap) continue;
         const int conc = std::min(nslots_, cap / (int)t.size());
         const int rounds = (nslots_ + conc - 1) / conc;
-        const double cost = rounds * (3.0 + 0.35 * shapes[i].rows);
-        if (res_.shape < 0 || cost < best) {
+        const double cost = rounds * shapes[i].us;
+        if (cost < best) {
             best = cost;
             res_.shape = i;
             res_.conc = conc;

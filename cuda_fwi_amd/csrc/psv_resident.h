@@ -49,9 +49,11 @@ struct ResidentParams {
 };
 
 // Tile shapes a launch can take: waves of a workgroup, stacked in z, and rows per wave of
-// the interior and of the edge tiles.
+// the interior and of the edge tiles; us: what a step takes (forward and adjoint mean, order
+// 4, one MI355X, a grid that fills the launch), for the choice among them.
 struct ResShape {
     int waves, rows, rows_edge;
+    double us;
 };
 
 // The shapes built for a type (sizeof(T) bytes per value), smallest first; returns their

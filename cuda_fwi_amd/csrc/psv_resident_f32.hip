@@ -5,15 +5,17 @@ namespace psv {
 
 namespace {
 
-const ResShape kShapes[] = {{8, 2, 2}, {16, 4, 3}, {16, 7, 4}};
+const ResShape kShapes[] = {{8, 2, 2, 3.8}, {12, 4, 3, 5.2}, {16, 4, 3, 5.8}, {12, 6, 4, 6.6}, {12, 9, 5, 12.5}};
 
 template <>
 const void* kernel_of<float>(int order, int mode, int shape, int* threads)
 {
-    if (shape >= 0 && shape < 3) *threads = kShapes[shape].waves * 64;
+    if (shape >= 0 && shape < 5) *threads = kShapes[shape].waves * 64;
     if (shape == 0) return resident_kernel<float, 8, 2, 2>(order, mode);
-    if (shape == 1) return resident_kernel<float, 16, 4, 3>(order, mode);
-    if (shape == 2) return resident_kernel<float, 16, 7, 4>(order, mode);
+    if (shape == 1) return resident_kernel<float, 12, 4, 3>(order, mode);
+    if (shape == 2) return resident_kernel<float, 16, 4, 3>(order, mode);
+    if (shape == 3) return resident_kernel<float, 12, 6, 4>(order, mode);
+    if (shape == 4) return resident_kernel<float, 12, 9, 5>(order, mode);
     return nullptr;
 }
 
@@ -23,7 +25,7 @@ template <>
 int resident_shapes<float>(const ResShape** out)
 {
     *out = kShapes;
-    return 3;
+    return 5;
 }
 
 template hipError_t resident_capacity<float>(int, int, int, int*);

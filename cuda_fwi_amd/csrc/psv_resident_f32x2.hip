@@ -7,14 +7,15 @@ namespace psv {
 
 namespace {
 
-const ResShape kShapes[] = {{8, 2, 2}, {16, 3, 2}};
+const ResShape kShapes[] = {{8, 2, 2, 12.5}, {12, 2, 2, 17}, {12, 3, 2, 20.5}};
 
 template <>
 const void* kernel_of<dfloat>(int order, int mode, int shape, int* threads)
 {
-    if (shape >= 0 && shape < 2) *threads = kShapes[shape].waves * 64;
+    if (shape >= 0 && shape < 3) *threads = kShapes[shape].waves * 64;
     if (shape == 0) return resident_kernel<dfloat, 8, 2, 2>(order, mode);
-    if (shape == 1) return resident_kernel<dfloat, 16, 3, 2>(order, mode);
+    if (shape == 1) return resident_kernel<dfloat, 12, 2, 2>(order, mode);
+    if (shape == 2) return resident_kernel<dfloat, 12, 3, 2>(order, mode);
     return nullptr;
 }
 
@@ -24,7 +25,7 @@ template <>
 int resident_shapes<dfloat>(const ResShape** out)
 {
     *out = kShapes;
-    return 2;
+    return 3;
 }
 
 template <>
