@@ -248,6 +248,8 @@ private:
     struct Resident {
         int slots = 0, shape = -1, conc = 0, waves = 0, rows = 0, rows_edge = 0, gen = 0;
         bool failed = false;    // refused or aborted once: the plan keeps to the split step
+        bool want = false;      // chosen for a plan with the exact gradient ...
+        bool discrete = false;  // ... and its shape has the replay and the reverse steps
         bool uploaded = false;
         int kdiv = 0;           // some CPML K differs from 1
         std::vector<psv::ResTile> h;
@@ -294,7 +296,8 @@ private:
                                 const Tables& tab, bool fwd_sig, hipGraphExec_t* out);
 
     // ------------------------------------------------------- plan_resident.cpp
-    std::vector<psv::ResTile> resident_tiles(const psv::ResShape& sh) const;
+    std::vector<psv::ResTile> resident_tiles(const psv::ResShape& sh, bool discrete) const;
+    size_t resident_terms() const;
     bool resident_ready();
     psvfwi_status resident_points(Tables& t);
     psvfwi_status resident_prepare();
@@ -515,6 +518,7 @@ private:
     hipEvent_t sample_ev_[kMaxSamples][3] = {};
     int samp_kind_[kMaxSamples] = {};
     int samp_steps_[kMaxSamples] = {};  // time steps the sample covers
+    bool samp_one_[kMaxSamples] = {};   // they are one kernel: no velocity kernel to time
     int nsamp_ = 0;
     double kus_[3][2] = {};
     int kn_[3] = {};

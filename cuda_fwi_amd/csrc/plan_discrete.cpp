@@ -5,8 +5,9 @@
 namespace psvplan {
 
 // Discrete gradient: per segment (last first), restore its checkpoint,
-// replay it keeping the state before every step and after the last, then
-// run the transposed steps back through it.  With segments of one step the
+// replay it keeping the state before every step and after the last (the
+// resident loop: the derivative terms of every step), then run the transposed
+// steps back through it.  With segments of one step the
 // forward kept every state, and the transposed steps read those directly.
 template <typename T>
 psvfwi_status Plan<T>::adjoint_discrete()
@@ -24,17 +25,28 @@ psvfwi_status Plan<T>::adjoint_discrete()
     PSV_TRY(alloc_state(adj_));
     PSV_TRY(zero_state(adj_));
     const size_t nf = (size_t)nslots_ * fst_;
-    for (int i = 0; i < 8; i++) {
-        PSV_HIP(dw_[i].alloc(nf));
-        PSV_HIP(psv::launch_fill<T>(dw_[i].p, nf, (T)0, stream_));
-    }
     for (int i = 0; i < 5; i++) {
         PSV_HIP(dg_[i].alloc(nf));
         PSV_HIP(psv::launch_fill<T>(dg_[i].p, nf, (T)0, stream_));
     }
     // segments of one step: the forward kept every state, no replay
     const bool every = kk == 1;
-    if (!every) {
+    bool resident = kk >= kResidentMin && resident_ready() && res_.discrete;
+    if (resident) {
+        PSV_TRY(resident_prepare());
+        PSV_TRY(alloc_state(replay_));
+        // (the terms of a segment may need more memory than its states: then the split step)
+        if (seg_.reserve((size_t)std::min(kk, ntmax_) * res_.conc * resident_terms()) != hipSuccess) {
+            (void)hipGetLastError();
+            resident = false;
+        }
+    }
+    if (!resident) PSV_TRY(ensure_all_tile_lists());
+    for (int i = 0; i < 8 && !resident; i++) {
+        PSV_HIP(dw_[i].alloc(nf));
+        PSV_HIP(psv::launch_fill<T>(dw_[i].p, nf, (T)0, stream_));
+    }
+    if (!every && !resident) {
         PSV_TRY(alloc_state(replay_));
         if (fused()) {
             PSV_TRY(alloc_state(replay2_));
@@ -78,13 +90,29 @@ psvfwi_status Plan<T>::adjoint_discrete()
     PSV_HIP(hipEventRecord(ev0_, stream_));
     launches_ = 0;
     AllSlotsAfter restore{this};
-    for (int w0 = 0; w0 < nslots_; w0 += group_size()) {
-        set_group(w0);
+    const int gsize = resident ? res_.conc : group_size();
+    for (int w0 = 0; w0 < nslots_; w0 += gsize) {
+        set_group(w0, gsize);
         const int ntg = group_nt();
         const int nseg = (ntg + kk - 1) / kk;
         for (int c = nseg - 1; c >= 0; c--) {
             const int t0 = c * kk, t1 = std::min(t0 + kk, ntg);
             // the states before steps t0 .. t1 - 1 and after t1 - 1
+            if (resident) {
+                PSV_TRY(restore_checkpoint(c, active(t0)));
+                PSV_TRY(launch_resident(replay_, fwd_tab_noreceivers_, true, psv::kReplay, -1, t0, t1, 0, 0));
+                // the shots that end in this segment start with their last step's sources
+                for (int it = t1 - 1; it >= t0; it--) {
+                    psv::DiscreteParams<T> d = dparams(it, View{}, View{});
+                    d.max_groups = maxg;
+                    d.inj_lo = active(it + 1);
+                    d.inj_hi = d.nslots;
+                    PSV_HIP(psv::launch_discrete_inject<T>(d, stream_));
+                }
+                PSV_TRY(launch_resident(adj_, adj_tab_, false, psv::kReverse, -1, t0, t1, 0, 0));
+                launches_ += 2 * (t1 - t0);
+                continue;
+            }
             const T* base = every ? ckpt_.p + (size_t)t0 * state_elems() : seg_.p;
             if (!every) {
                 PSV_TRY(restore_checkpoint(c, active(t0)));
@@ -120,6 +148,7 @@ psvfwi_status Plan<T>::adjoint_discrete()
     all_slots();
     PSV_HIP(hipEventRecord(ev1_, stream_));
     PSV_HIP(hipStreamSynchronize(stream_));
+    if (resident && resident_failed()) return adjoint_discrete();
     float ms = 0;
     PSV_HIP(hipEventElapsedTime(&ms, ev0_, ev1_));
     last_ms_ = ms;

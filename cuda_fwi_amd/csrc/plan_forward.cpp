@@ -43,8 +43,7 @@ psvfwi_status Plan<T>::forward(int flags)
     if (snap) PSV_HIP(snaps_.alloc((size_t)((ntmax_ - 1) / snap_interval_ + 1) * nslots_ * fst_));
     snaps_taken_ = snap;
 
-    // (the discrete adjoint replays with the split step)
-    if (!resident || discrete) PSV_TRY(ensure_all_tile_lists());
+    if (!resident) PSV_TRY(ensure_all_tile_lists());
     PSV_TRY(begin_samples());
     PSV_HIP(hipEventRecord(ev0_, stream_));
     launches_ = 0;

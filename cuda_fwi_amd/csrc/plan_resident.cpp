@@ -8,10 +8,9 @@ namespace psvplan {
 
 namespace {
 
-// The rows of one column of tiles.  A tile is interior when every stress cell it computes
-// (2 cells around the owned ones) is updated, outside the CPML strips and below the
-// free-surface row: rows in [zlo, zhi) (and xin, the same in x).  Interior tiles take up to
-// `own` rows, edge tiles up to `own_edge`; the fewest tiles that cover the column.
+// The rows of one column of tiles.  A tile is interior when the rows it owns are in
+// [zlo, zhi) (and xin, the same in x).  Interior tiles take up to `own` rows, edge tiles up to
+// `own_edge`; the fewest tiles that cover the column.
 void tile_column(int nzt, int zlo, int zhi, bool xin, int own, int own_edge, int x0, int x1, int xr,
                  std::vector<psv::ResTile>& out)
 {
@@ -21,8 +20,8 @@ void tile_column(int nzt, int zlo, int zhi, bool xin, int own, int own_edge, int
         const int he = std::min(own_edge, nzt - z);
         need[(size_t)z] = 1 + need[(size_t)(z + he)];
         step[(size_t)z] = he;
-        const int hi = std::min(own, zhi - 2 - z);
-        if (xin && z - 2 >= zlo && hi > 0 && 1 + need[(size_t)(z + hi)] <= need[(size_t)z]) {
+        const int hi = std::min(own, zhi - z);
+        if (xin && z >= zlo && hi > 0 && 1 + need[(size_t)(z + hi)] <= need[(size_t)z]) {
             need[(size_t)z] = 1 + need[(size_t)(z + hi)];
             step[(size_t)z] = -hi;
         }
@@ -44,15 +43,24 @@ void tile_column(int nzt, int zlo, int zhi, bool xin, int own, int own_edge, int
 
 }  // namespace
 
-// The tiles of the grid for a shape.
+// The tiles of the grid for a shape.  Interior tiles: every stress cell they compute (2 cells
+// around the owned ones) is updated, outside the CPML strips and below the free-surface row;
+// for the transposed steps also every velocity weight they form (4 cells around) is one of an
+// updated cell outside the strips, and none of their stress cells is mirrored.
 template <typename T>
-std::vector<psv::ResTile> Plan<T>::resident_tiles(const psv::ResShape& sh) const
+std::vector<psv::ResTile> Plan<T>::resident_tiles(const psv::ResShape& sh, bool discrete) const
 {
     const int nzt = g_.nzt, nxt = g_.nxt, H = fpad_;
     const bool pml = g_.npml > 0;
-    const int zlo = g_.fsurf ? H + 1 : (pml ? ppad_ + 1 : H);
-    const int zhi = pml ? nzt - ppad_ - 1 : nzt - H;
-    const int xlo = pml ? ppad_ + 1 : H, xhi = pml ? nxt - ppad_ - 1 : nxt - H;
+    int zlo = 2 + (g_.fsurf ? H + 1 : (pml ? ppad_ + 1 : H));
+    int zhi = (pml ? nzt - ppad_ - 1 : nzt - H) - 2;
+    int xlo = 2 + (pml ? ppad_ + 1 : H), xhi = (pml ? nxt - ppad_ - 1 : nxt - H) - 2;
+    if (discrete) {
+        zlo = std::max(zlo, g_.fsurf ? 2 * H + 3 : 4 + (pml ? ppad_ : H));
+        xlo = std::max(xlo, 4 + (pml ? ppad_ : H));
+        zhi -= 2;
+        xhi -= 2;
+    }
     const int own = sh.rows * sh.waves - 2 * psv::kResHalo;
     const int own_edge = sh.rows_edge * sh.waves - 2 * psv::kResHalo;
     std::vector<psv::ResTile> out;
@@ -64,9 +72,14 @@ std::vector<psv::ResTile> Plan<T>::resident_tiles(const psv::ResShape& sh) const
         const int left = ncol - 1 - c, rest = left == 0 ? 0 : (left - 1) * W + end;
         const int most = ncol == 1 ? 64 : (c == 0 || left == 0 ? end : W);
         const int x1 = x + std::min(most, std::max((nxt - x + left) / (left + 1), nxt - x - rest));
-        const bool xin = x - 2 >= xlo && x1 + 2 <= xhi;
+        const bool xin = x >= xlo && x1 <= xhi;
         tile_column(nzt, zlo, zhi, xin, own, own_edge, x, x1, std::max(0, x - psv::kResHalo), out);
         x = x1;
+    }
+    int rows = 0;
+    for (psv::ResTile& t : out) {
+        t.row0 = rows;
+        rows += sh.waves * (t.edge ? sh.rows_edge : sh.rows);
     }
     return out;
 }
@@ -97,30 +110,38 @@ bool Plan<T>::resident_ready()
     }
     // every tile needs room for the mirror rows and the rim of a neighbour
     if (g_.nxt < 16 || g_.nzt < 16) return false;
-    if (res_.slots == nslots_) return res_.shape >= 0;
+    const bool want = grad_mode_ == PSVFWI_GRADIENT_DISCRETE;
+    if (res_.slots == nslots_ && res_.want == want) return res_.shape >= 0;
     res_.slots = nslots_;
+    res_.want = want;
     res_.shape = -1;
-    // the shots run conc at a time, rounds times over; the split step takes them together
-    double best = split_step_us((double)nslots_ * g_.nzt * g_.nxt, (int)sizeof(T), std::is_same<T, psv::dfloat>::value);
-    for (int i = 0; i < n; i++) {
-        const std::vector<psv::ResTile> t = resident_tiles(shapes[i]);
-        int cap = 1 << 30;
-        for (int mode : {(int)psv::kForward, (int)psv::kAdjoint}) {
-            int c = 0;
-            if (psv::resident_capacity<T>(g_.fdorder, mode, i, &c) != hipSuccess) c = 0;
-            cap = std::min(cap, c);
-        }
-        if ((int)t.size() > cap) continue;
-        const int conc = std::min(nslots_, cap / (int)t.size());
-        const int rounds = (nslots_ + conc - 1) / conc;
-        const double cost = rounds * shapes[i].us;
-        if (cost < best) {
-            best = cost;
-            res_.shape = i;
-            res_.conc = conc;
-            res_.h = t;
+    // with the exact gradient, a shape that has the replay and the reverse steps; without one,
+    // a shape for the forward runs only
+    for (int d = want; d >= 0 && res_.shape < 0; d--) {
+        // the shots run conc at a time, rounds times over; the split step takes them together
+        double best = split_step_us((double)nslots_ * g_.nzt * g_.nxt, (int)sizeof(T), std::is_same<T, psv::dfloat>::value);
+        for (int i = 0; i < n; i++) {
+            const std::vector<psv::ResTile> t = resident_tiles(shapes[i], d != 0);
+            int cap = 1 << 30;
+            for (int mode = psv::kForward; mode <= (d ? psv::kReverse : (int)psv::kAdjoint); mode++) {
+                int c = 0;
+                if (psv::resident_capacity<T>(g_.fdorder, mode, i, &c) != hipSuccess) c = 0;
+                cap = std::min(cap, c);
+            }
+            if ((int)t.size() > cap) continue;
+            const int conc = std::min(nslots_, cap / (int)t.size());
+            const int rounds = (nslots_ + conc - 1) / conc;
+            const double cost = rounds * shapes[i].us;
+            if (cost < best) {
+                best = cost;
+                res_.shape = i;
+                res_.conc = conc;
+                res_.h = t;
+                res_.discrete = d != 0;
+            }
         }
     }
+    (void)hipGetLastError();  // a shape that is not built is no error
     if (res_.shape < 0) return false;
     res_.waves = shapes[res_.shape].waves;
     res_.rows = shapes[res_.shape].rows;
@@ -232,6 +253,12 @@ psvfwi_status Plan<T>::launch_resident(State<T>& st, Tables& tab, bool fwd_sig, 
         res_.tag = 1;
     }
     psv::ResidentParams<T> a{};
+    if (mode >= psv::kReplay) {
+        a.terms = seg_.p;
+        a.terms_slot = resident_terms();
+        a.terms_step = a.terms_slot * (size_t)res_.conc;
+        for (int i = 0; i < 5; i++) a.g5[i] = atw(dg_[i], fst_);
+    }
     a.p = base_params(st, tab, fwd_sig);
     a.p.nslots = active(it0);
     a.p.flags = flags;
@@ -263,13 +290,21 @@ psvfwi_status Plan<T>::launch_resident(State<T>& st, Tables& tab, bool fwd_sig, 
     }
     if (sample) {
         PSV_HIP(hipEventRecord(sample_ev_[nsamp_][1], stream_));
-        PSV_HIP(hipEventRecord(sample_ev_[nsamp_][2], stream_));
         samp_kind_[nsamp_] = kind;
         samp_steps_[nsamp_] = steps;
+        samp_one_[nsamp_] = true;
         nsamp_++;
     }
     if (kind >= 0) launches_ += steps;
     return PSVFWI_OK;
+}
+
+// Elements of one step's derivative terms of a slot.
+template <typename T>
+size_t Plan<T>::resident_terms() const
+{
+    const psv::ResTile& t = res_.h.back();
+    return (size_t)(t.row0 + res_.waves * (t.edge ? res_.rows_edge : res_.rows)) * 320;
 }
 
 // After the stream has drained: a resident run whose waits ran out, or that was refused,
@@ -284,8 +319,9 @@ bool Plan<T>::resident_failed()
 }
 
 #define PSV_INSTANTIATE(T) \
-    template std::vector<psv::ResTile> Plan<T>::resident_tiles(const psv::ResShape&) const; \
+    template std::vector<psv::ResTile> Plan<T>::resident_tiles(const psv::ResShape&, bool) const; \
     template bool Plan<T>::resident_ready(); \
+    template size_t Plan<T>::resident_terms() const; \
     template psvfwi_status Plan<T>::resident_points(Tables&); \
     template psvfwi_status Plan<T>::resident_prepare(); \
     template psvfwi_status Plan<T>::launch_resident(State<T>&, Tables&, bool, int, int, int, int, int, int, bool); \

@@ -228,6 +228,7 @@ psvfwi_status Plan<T>::launch_timed(const psv::StepParams<T>& p, int mode, int k
         PSV_HIP(hipEventRecord(sample_ev_[nsamp_][2], stream_));
         samp_kind_[nsamp_] = kind;
         samp_steps_[nsamp_] = 1;
+        samp_one_[nsamp_] = false;
         nsamp_++;
     } else {
         PSV_TRY(launch_plain(p, mode, st, alt));
@@ -257,7 +258,7 @@ psvfwi_status Plan<T>::collect_samples()
             if (samp_kind_[i] != k) continue;
             float m1 = 0, m2 = 0;
             PSV_HIP(hipEventElapsedTime(&m1, sample_ev_[i][0], sample_ev_[i][1]));
-            PSV_HIP(hipEventElapsedTime(&m2, sample_ev_[i][1], sample_ev_[i][2]));
+            if (!samp_one_[i]) PSV_HIP(hipEventElapsedTime(&m2, sample_ev_[i][1], sample_ev_[i][2]));
             a += m1 / samp_steps_[i];
             b += m2 / samp_steps_[i];
             n++;

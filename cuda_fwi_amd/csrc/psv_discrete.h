@@ -77,6 +77,9 @@ struct DiscreteParams {
 // stress pass (gather, transposed mirror, stress weights, and the next step's
 // receiver sources).  The velocity adjoints gathered from the last step's
 // stress weights are never added: nothing reads them.
+// (launch_discrete_inject: the receiver kernel alone)
+template <typename T>
+hipError_t launch_discrete_inject(const DiscreteParams<T>& p, hipStream_t s);
 template <typename T>
 hipError_t launch_discrete_step(const DiscreteParams<T>& p, int order, hipStream_t s);
 

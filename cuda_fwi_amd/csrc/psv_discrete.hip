@@ -422,14 +422,25 @@ __global__ __launch_bounds__(kDX* kDZ) void d_stress_pass_kernel(const DiscreteP
     p.ws3[k] = w_vz_z;
 }
 
+}  // namespace
+
+template <typename T>
+hipError_t launch_discrete_inject(const DiscreteParams<T>& p, hipStream_t s)
+{
+    if (p.max_groups <= 0 || p.inj_hi <= p.inj_lo) return hipSuccess;
+    hipLaunchKernelGGL((d_inject_kernel<T>), dim3((p.max_groups + 63) / 64, p.inj_hi - p.inj_lo), dim3(64), 0, s, p);
+    return hipGetLastError();
+}
+
+namespace {
+
 template <typename T, int ORDER>
 hipError_t discrete_step(const DiscreteParams<T>& p, hipStream_t s)
 {
     const dim3 blk(kDX, kDZ);
     const dim3 grd((p.nxt + kDX - 1) / kDX, (p.nzt + kDZ - 1) / kDZ, p.nslots);
-    if (p.max_groups > 0 && p.inj_hi > p.inj_lo)
-        hipLaunchKernelGGL((d_inject_kernel<T>), dim3((p.max_groups + 63) / 64, p.inj_hi - p.inj_lo),
-                           dim3(64), 0, s, p);
+    const hipError_t e = launch_discrete_inject<T>(p, s);
+    if (e != hipSuccess) return e;
     hipLaunchKernelGGL((d_vel_pass_kernel<T, ORDER>), grd, blk, 0, s, p);
     hipLaunchKernelGGL((d_stress_pass_kernel<T, ORDER>), grd, blk, 0, s, p);
     return hipGetLastError();
@@ -446,6 +457,10 @@ hipError_t launch_discrete_step(const DiscreteParams<T>& p, int order, hipStream
     return hipErrorInvalidValue;
 }
 
+template hipError_t launch_discrete_inject<float>(const DiscreteParams<float>&, hipStream_t);
+template hipError_t launch_discrete_inject<double>(const DiscreteParams<double>&, hipStream_t);
+template hipError_t launch_discrete_inject<dfloat>(const DiscreteParams<dfloat>&, hipStream_t);
+template hipError_t launch_discrete_inject<ffloat>(const DiscreteParams<ffloat>&, hipStream_t);
 template hipError_t launch_discrete_step<float>(const DiscreteParams<float>&, int, hipStream_t);
 template hipError_t launch_discrete_step<double>(const DiscreteParams<double>&, int, hipStream_t);
 template hipError_t launch_discrete_step<dfloat>(const DiscreteParams<dfloat>&, int, hipStream_t);

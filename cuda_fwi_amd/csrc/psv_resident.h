@@ -18,7 +18,7 @@ struct ResTile {
     int z0, z1, x0, x1;
     int zr, xr;
     int edge;  // the region meets a CPML strip, the free surface or the grid's frame
-    int pad;
+    int row0;  // rows of all waves of the tiles before this one
 };
 
 // Point sources and receivers of a (slot, tile, wave): layers of at most one entry per
@@ -29,6 +29,11 @@ struct ResPoints {
     const int* head;
     const int* id;    // [layer][64]
 };
+
+// What a launch runs: the forward and adjoint steps (kForward, kAdjoint), and for the exact
+// gradient a forward segment that writes its derivative terms and the transposed steps that
+// read them back.
+enum { kReplay = 2, kReverse = 3 };
 
 template <typename T>
 struct ResidentParams {
@@ -46,7 +51,17 @@ struct ResidentParams {
     unsigned tag;            // tag of the launch's first step
     int* aborted;            // host memory: set when a wait ran out
     int kdiv;                // some CPML K differs from 1
+    // replay and reverse: five values per cell, [step - it0][slot][row of a wave][5][64 lanes],
+    // and the reverse steps' gradients (lam, mu, mu_zx, rho_zp, rho_xp)
+    T* terms;
+    size_t terms_step, terms_slot;
+    T* g5[5];
 };
+
+// The tile shapes (ResShape) of each type: X(index, waves, rows, rows_edge, us)
+#define PSV_RESIDENT_F32(X) X(0, 8, 2, 2, 3.8) X(1, 12, 4, 3, 5.2) X(2, 16, 4, 3, 5.8) X(3, 12, 6, 4, 6.6) X(4, 12, 9, 5, 12.5)
+#define PSV_RESIDENT_F64(X) X(0, 8, 2, 2, 5.6) X(1, 12, 2, 2, 7.2) X(2, 8, 4, 3, 7.6) X(3, 12, 3, 2, 8.8) X(4, 12, 4, 3, 14.5)
+#define PSV_RESIDENT_F32X2(X) X(0, 8, 2, 2, 12.5) X(1, 12, 2, 2, 17) X(2, 12, 3, 2, 20.5)
 
 // Tile shapes a launch can take: waves of a workgroup, stacked in z, and rows per wave of
 // the interior and of the edge tiles; us: what a step takes (forward and adjoint mean, order
@@ -60,6 +75,13 @@ struct ResShape {
 // number (0: the type has no resident loop).
 template <typename T>
 int resident_shapes(const ResShape** out);
+
+// The kernel of an order, mode and shape and its workgroup size (null: not built): forward and
+// adjoint, replay and reverse.
+template <typename T>
+const void* resident_kernel(int order, int mode, int shape, int* threads);
+template <typename T>
+const void* resident_kernel_discrete(int order, int mode, int shape, int* threads);
 
 // Workgroups of one launch that are resident together on the current device.
 template <typename T>

@@ -1,31 +1,28 @@
 // psv_resident_f32.hip -- the resident time loop in FP32.
 #include "psv_resident.inc"
+#include "psv_resident_launch.inc"
 
 namespace psv {
-
-namespace {
-
-const ResShape kShapes[] = {{8, 2, 2, 3.8}, {12, 4, 3, 5.2}, {16, 4, 3, 5.8}, {12, 6, 4, 6.6}, {12, 9, 5, 12.5}};
-
-template <>
-const void* kernel_of<float>(int order, int mode, int shape, int* threads)
-{
-    if (shape >= 0 && shape < 5) *threads = kShapes[shape].waves * 64;
-    if (shape == 0) return resident_kernel<float, 8, 2, 2>(order, mode);
-    if (shape == 1) return resident_kernel<float, 12, 4, 3>(order, mode);
-    if (shape == 2) return resident_kernel<float, 16, 4, 3>(order, mode);
-    if (shape == 3) return resident_kernel<float, 12, 6, 4>(order, mode);
-    if (shape == 4) return resident_kernel<float, 12, 9, 5>(order, mode);
-    return nullptr;
-}
-
-}  // namespace
 
 template <>
 int resident_shapes<float>(const ResShape** out)
 {
-    *out = kShapes;
-    return 5;
+#define PSV_SHAPE(I, NW, R, RE, US) {NW, R, RE, US},
+    static const ResShape shapes[] = {PSV_RESIDENT_F32(PSV_SHAPE)};
+    *out = shapes;
+    return (int)(sizeof shapes / sizeof shapes[0]);
+}
+
+template <>
+const void* resident_kernel<float>(int order, int mode, int shape, int* threads)
+{
+#define PSV_KERNEL(I, NW, R, RE, US) \
+    if (shape == I) { \
+        *threads = NW * 64; \
+        return kernel_of<float, kForward, kAdjoint, NW, R, RE>(order, mode); \
+    }
+    PSV_RESIDENT_F32(PSV_KERNEL)
+    return nullptr;
 }
 
 template hipError_t resident_capacity<float>(int, int, int, int*);

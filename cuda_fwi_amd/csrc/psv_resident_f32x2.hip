@@ -2,31 +2,33 @@
 // contraction has none: what the compiler fuses depends on the code around it, so another
 // kernel would give other roundings than the split step's.
 #include "psv_resident.inc"
+#include "psv_resident_launch.inc"
 
 namespace psv {
-
-namespace {
-
-const ResShape kShapes[] = {{8, 2, 2, 12.5}, {12, 2, 2, 17}, {12, 3, 2, 20.5}};
-
-template <>
-const void* kernel_of<dfloat>(int order, int mode, int shape, int* threads)
-{
-    if (shape >= 0 && shape < 3) *threads = kShapes[shape].waves * 64;
-    if (shape == 0) return resident_kernel<dfloat, 8, 2, 2>(order, mode);
-    if (shape == 1) return resident_kernel<dfloat, 12, 2, 2>(order, mode);
-    if (shape == 2) return resident_kernel<dfloat, 12, 3, 2>(order, mode);
-    return nullptr;
-}
-
-}  // namespace
 
 template <>
 int resident_shapes<dfloat>(const ResShape** out)
 {
-    *out = kShapes;
-    return 3;
+#define PSV_SHAPE(I, NW, R, RE, US) {NW, R, RE, US},
+    static const ResShape shapes[] = {PSV_RESIDENT_F32X2(PSV_SHAPE)};
+    *out = shapes;
+    return (int)(sizeof shapes / sizeof shapes[0]);
 }
+
+template <>
+const void* resident_kernel<dfloat>(int order, int mode, int shape, int* threads)
+{
+#define PSV_KERNEL(I, NW, R, RE, US) \
+    if (shape == I) { \
+        *threads = NW * 64; \
+        return kernel_of<dfloat, kForward, kAdjoint, NW, R, RE>(order, mode); \
+    }
+    PSV_RESIDENT_F32X2(PSV_KERNEL)
+    return nullptr;
+}
+
+template hipError_t resident_capacity<dfloat>(int, int, int, int*);
+template hipError_t launch_resident<dfloat>(const ResidentParams<dfloat>&, int, int, int, hipStream_t);
 
 template <>
 int resident_shapes<ffloat>(const ResShape** out)
@@ -46,8 +48,5 @@ hipError_t launch_resident<ffloat>(const ResidentParams<ffloat>&, int, int, int,
 {
     return hipErrorInvalidValue;
 }
-
-template hipError_t resident_capacity<dfloat>(int, int, int, int*);
-template hipError_t launch_resident<dfloat>(const ResidentParams<dfloat>&, int, int, int, hipStream_t);
 
 }  // namespace psv

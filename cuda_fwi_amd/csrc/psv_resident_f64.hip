@@ -1,31 +1,28 @@
 // psv_resident_f64.hip -- the resident time loop in FP64.
 #include "psv_resident.inc"
+#include "psv_resident_launch.inc"
 
 namespace psv {
-
-namespace {
-
-const ResShape kShapes[] = {{8, 2, 2, 5.6}, {12, 2, 2, 7.2}, {8, 4, 3, 7.6}, {12, 3, 2, 8.8}, {12, 4, 3, 14.5}};
-
-template <>
-const void* kernel_of<double>(int order, int mode, int shape, int* threads)
-{
-    if (shape >= 0 && shape < 5) *threads = kShapes[shape].waves * 64;
-    if (shape == 0) return resident_kernel<double, 8, 2, 2>(order, mode);
-    if (shape == 1) return resident_kernel<double, 12, 2, 2>(order, mode);
-    if (shape == 2) return resident_kernel<double, 8, 4, 3>(order, mode);
-    if (shape == 3) return resident_kernel<double, 12, 3, 2>(order, mode);
-    if (shape == 4) return resident_kernel<double, 12, 4, 3>(order, mode);
-    return nullptr;
-}
-
-}  // namespace
 
 template <>
 int resident_shapes<double>(const ResShape** out)
 {
-    *out = kShapes;
-    return 5;
+#define PSV_SHAPE(I, NW, R, RE, US) {NW, R, RE, US},
+    static const ResShape shapes[] = {PSV_RESIDENT_F64(PSV_SHAPE)};
+    *out = shapes;
+    return (int)(sizeof shapes / sizeof shapes[0]);
+}
+
+template <>
+const void* resident_kernel<double>(int order, int mode, int shape, int* threads)
+{
+#define PSV_KERNEL(I, NW, R, RE, US) \
+    if (shape == I) { \
+        *threads = NW * 64; \
+        return kernel_of<double, kForward, kAdjoint, NW, R, RE>(order, mode); \
+    }
+    PSV_RESIDENT_F64(PSV_KERNEL)
+    return nullptr;
 }
 
 template hipError_t resident_capacity<double>(int, int, int, int*);
