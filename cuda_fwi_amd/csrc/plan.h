@@ -256,7 +256,7 @@ private:
         DBuf<psv::ResTile> tiles;
         DBuf<unsigned long long> exch;
         size_t exch_slot = 0;
-        int xpitch = 0;
+        int xpitch = 0, zpitch = 0;
         unsigned tag = 1;
         int* aborted = nullptr;  // pinned host memory the kernel writes when a wait runs out
     };

@@ -45,7 +45,7 @@ void tile_column(int nzt, int zlo, int zhi, bool xin, int own, int own_edge, int
 
 // The tiles of the grid for a shape.  Interior tiles: every stress cell they compute (2 cells
 // around the owned ones) is updated, outside the CPML strips and below the free-surface row;
-// for the transposed steps also every velocity weight they form (4 cells around) is one of an
+// for the transposed steps also every velocity weight they form (kResHalo cells around) is one of an
 // updated cell outside the strips, and none of their stress cells is mirrored.
 template <typename T>
 std::vector<psv::ResTile> Plan<T>::resident_tiles(const psv::ResShape& sh, bool discrete) const
@@ -56,10 +56,10 @@ std::vector<psv::ResTile> Plan<T>::resident_tiles(const psv::ResShape& sh, bool 
     int zhi = (pml ? nzt - ppad_ - 1 : nzt - H) - 2;
     int xlo = 2 + (pml ? ppad_ + 1 : H), xhi = (pml ? nxt - ppad_ - 1 : nxt - H) - 2;
     if (discrete) {
-        zlo = std::max(zlo, g_.fsurf ? 2 * H + 3 : 4 + (pml ? ppad_ : H));
-        xlo = std::max(xlo, 4 + (pml ? ppad_ : H));
-        zhi -= 2;
-        xhi -= 2;
+        zlo = std::max(zlo, g_.fsurf ? 2 * H + 3 : psv::kResHalo + (pml ? ppad_ : H));
+        xlo = std::max(xlo, psv::kResHalo + (pml ? ppad_ : H));
+        zhi -= psv::kResHalo - 2;
+        xhi -= psv::kResHalo - 2;
     }
     const int own = sh.rows * sh.waves - 2 * psv::kResHalo;
     const int own_edge = sh.rows_edge * sh.waves - 2 * psv::kResHalo;
@@ -226,7 +226,8 @@ psvfwi_status Plan<T>::resident_prepare()
         res_.uploaded = true;
     }
     res_.xpitch = (int)round_up((size_t)g_.nxt, 8);
-    res_.exch_slot = (size_t)2 * g_.nzt * res_.xpitch * (2 * sizeof(T) / 4);
+    res_.zpitch = (int)round_up((size_t)g_.nzt, 8);
+    res_.exch_slot = 2 * ((size_t)g_.nzt * res_.xpitch + (size_t)g_.nxt * res_.zpitch) * (2 * sizeof(T) / 4);
     const size_t need = res_.exch_slot * (size_t)res_.conc;
     if (!res_.exch.p || res_.exch.cap < need) {
         PSV_HIP(res_.exch.alloc(need));
@@ -275,6 +276,7 @@ psvfwi_status Plan<T>::launch_resident(State<T>& st, Tables& tab, bool fwd_sig, 
     a.exch = res_.exch.p;
     a.exch_slot = res_.exch_slot;
     a.xpitch = res_.xpitch;
+    a.zpitch = res_.zpitch;
     a.tag = res_.tag;
     a.aborted = res_.aborted;
     a.kdiv = res_.kdiv;

@@ -9,7 +9,9 @@
 
 namespace psv {
 
-constexpr int kResHalo = 4;                    // velocity halo of a tile: two half-steps of two cells
+// Velocity halo of a tile.  Two half-steps reach four cells, but not in one direction: where the
+// staggered difference of one half reaches two cells the other's reaches one.
+constexpr int kResHalo = 3;
 constexpr int kResOwnX = 64 - 2 * kResHalo;    // columns a tile owns between two others
 
 // One workgroup's tile: it owns the cells [z0, z1) x [x0, x1) and holds the region
@@ -43,11 +45,11 @@ struct ResidentParams {
     int it0, it1;            // steps [it0, it1), each slot up to its own nt
     ResPoints pts;
     size_t tf_stride;        // elements from one stored time to the next
-    // velocity exchange: per slot two generations of [nzt][xpitch] cells, each value a
-    // 64-bit word {tag, 32 bits of the value}
+    // velocity exchange: per slot two generations of [nzt][xpitch] cells for the rims' rows and
+    // [nxt][zpitch] for their columns, every 32 bits of a value a 64-bit word with a tag
     unsigned long long* exch;
     size_t exch_slot;        // words per slot
-    int xpitch;
+    int xpitch, zpitch;
     unsigned tag;            // tag of the launch's first step
     int* aborted;            // host memory: set when a wait ran out
     int kdiv;                // some CPML K differs from 1
