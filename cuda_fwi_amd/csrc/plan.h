@@ -246,7 +246,7 @@ private:
     // the resident time loop (plan_resident.cpp): the tiles chosen for a batch of `slots`
     // shots (shape < 0: it does not fit), conc slots per launch
     struct Resident {
-        int slots = 0, shape = -1, conc = 0, waves = 0, rows = 0, rows_edge = 0, gen = 0;
+        int slots = 0, shape = -1, conc = 0, cap = 0, waves = 0, rows = 0, rows_edge = 0, gen = 0;
         bool failed = false;    // refused or aborted once: the plan keeps to the split step
         bool want = false;      // chosen for a plan with the exact gradient ...
         bool discrete = false;  // ... and its shape has the replay and the reverse steps
@@ -296,7 +296,7 @@ private:
                                 const Tables& tab, bool fwd_sig, hipGraphExec_t* out);
 
     // ------------------------------------------------------- plan_resident.cpp
-    std::vector<psv::ResTile> resident_tiles(const psv::ResShape& sh, bool discrete) const;
+    std::vector<psv::ResTile> resident_tiles(const psv::ResShape& sh, bool discrete, int most_rows) const;
     size_t resident_terms() const;
     bool resident_ready();
     psvfwi_status resident_points(Tables& t);

@@ -65,7 +65,8 @@ psvfwi_status Plan<T>::autotune(int steps, int* best)
     const int cand[kNumCand] = {4, 8, 16, 32, -8, -16, -32, -64};
     float best_ms = 1e30f;
     int best_tz = tz_;
-    // the resident loop first, where it fits
+    // the resident loop first, where it fits: over four times the steps, of which a launch's
+    // reading and writing of the state is a small part, as in a run
     float res_ms = 1e30f;
     tile_auto_ = true;
     if (resident_ready()) {
@@ -75,9 +76,12 @@ psvfwi_status Plan<T>::autotune(int steps, int* best)
         for (int rep = 0; rep < 2; rep++) {
             PSV_TRY(zero_state(main_));
             PSV_HIP(hipEventRecord(ev0_, stream_));
+            int split_steps = 0, res_steps = 0;
             for (int w0 = 0; w0 < nslots_; w0 += res_.conc) {
                 set_group(w0, res_.conc);
-                const int nstep = std::min(steps, group_nt());
+                const int nstep = std::min(4 * steps, group_nt());
+                split_steps += std::min(steps, group_nt());
+                res_steps += nstep;
                 PSV_TRY(launch_resident(main_, fwd_tab_noreceivers_, true, psv::kForward, -1, 0, nstep, 0, 0));
                 if (adj)
                     PSV_TRY(launch_resident(main_, adj_tab_, false, psv::kAdjoint, -1, 0, nstep, psv::kStore, 0, true));
@@ -86,6 +90,7 @@ psvfwi_status Plan<T>::autotune(int steps, int* best)
             PSV_HIP(hipEventRecord(ev1_, stream_));
             PSV_HIP(hipStreamSynchronize(stream_));
             PSV_HIP(hipEventElapsedTime(&res_ms, ev0_, ev1_));
+            res_ms *= (float)split_steps / res_steps;
         }
         if (resident_failed()) res_ms = 1e30f;
     }

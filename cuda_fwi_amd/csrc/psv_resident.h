@@ -60,10 +60,15 @@ struct ResidentParams {
     T* g5[5];
 };
 
-// The tile shapes (ResShape) of each type: X(index, waves, rows, rows_edge, us)
-#define PSV_RESIDENT_F32(X) X(0, 8, 2, 2, 3.8) X(1, 12, 4, 3, 5.2) X(2, 16, 4, 3, 5.8) X(3, 12, 6, 4, 6.6) X(4, 12, 9, 5, 12.5)
-#define PSV_RESIDENT_F64(X) X(0, 8, 2, 2, 5.6) X(1, 12, 2, 2, 7.2) X(2, 8, 4, 3, 7.6) X(3, 12, 3, 2, 8.8) X(4, 12, 4, 3, 14.5)
-#define PSV_RESIDENT_F32X2(X) X(0, 8, 2, 2, 12.5) X(1, 12, 2, 2, 17) X(2, 12, 3, 2, 20.5)
+// The tile shapes (ResShape) of each type: X(index, waves, rows, rows_edge, us).  12 waves have
+// 168 registers each and 8 have 256, which hold about 9 rows of FP32 and 6 of the 8-byte types.
+#define PSV_RESIDENT_F32(X)                                                                        \
+    X(0, 8, 2, 2, 2.9) X(1, 8, 3, 2, 3.3) X(2, 12, 3, 2, 3.5) X(3, 12, 4, 3, 4.0) X(4, 12, 5, 4, 4.7) \
+    X(5, 12, 6, 4, 5.2) X(6, 12, 7, 5, 6.0) X(7, 12, 8, 5, 7.0) X(8, 12, 9, 5, 7.6)
+#define PSV_RESIDENT_F64(X)                                                                        \
+    X(0, 8, 2, 2, 3.4) X(1, 8, 3, 2, 4.4) X(2, 12, 3, 2, 5.0) X(3, 8, 4, 3, 5.3) X(4, 8, 6, 4, 7.3)   \
+    X(5, 8, 9, 5, 16.5)
+#define PSV_RESIDENT_F32X2(X) X(0, 8, 2, 2, 9.0) X(1, 8, 3, 2, 13.7) X(2, 12, 2, 2, 14.2) X(3, 8, 4, 3, 17.2)
 
 // Tile shapes a launch can take: waves of a workgroup, stacked in z, and rows per wave of
 // the interior and of the edge tiles; us: what a step takes (forward and adjoint mean, order
