@@ -298,6 +298,7 @@ private:
     // ------------------------------------------------------- plan_resident.cpp
     std::vector<psv::ResTile> resident_tiles(const psv::ResShape& sh, bool discrete, int most_rows) const;
     size_t resident_terms() const;
+    bool chain_upload() const;
     bool resident_ready();
     psvfwi_status resident_points(Tables& t);
     psvfwi_status resident_prepare();
@@ -505,6 +506,11 @@ private:
     DBuf<int> dgrp_off_, dblk_off_, dblk_idx_;
     int dnblk_ = 0;
     std::vector<double> h_pml_, h_mu_, h_mu_zx_, h_rho_zp_, h_rho_xp_;
+    // the model's mu, mu_zx, rho_zp, rho_xp in FP64 on the device, for the exact model gradient
+    // (uploaded after set_model when one is first taken), and that gradient
+    mutable DBuf<double> chain_model_, chain_out_;
+    mutable DBuf<int> chain_order_;
+    mutable bool chain_fresh_ = false;
     bool have_obs_ = false;
 
     // timing: the last run, and kernel samples every kSampleEvery-th launch

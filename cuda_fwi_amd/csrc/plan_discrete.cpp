@@ -147,6 +147,7 @@ psvfwi_status Plan<T>::adjoint_discrete()
     }
     all_slots();
     PSV_HIP(hipEventRecord(ev1_, stream_));
+    (void)chain_upload();  // while the steps run
     PSV_HIP(hipStreamSynchronize(stream_));
     if (resident && resident_failed()) return adjoint_discrete();
     float ms = 0;
@@ -287,11 +288,48 @@ psvfwi_status Plan<T>::get_coefficient_gradient(int shot, double* gl, double* gm
     return PSVFWI_OK;
 }
 
+// The FP64 model arrays that the chain rule from the coefficients to the model needs; false
+// where there is no memory for them.
+template <typename T>
+bool Plan<T>::chain_upload() const
+{
+    if (chain_fresh_) return true;
+    const std::vector<double>* a[4] = {&h_mu_, &h_mu_zx_, &h_rho_zp_, &h_rho_xp_};
+    size_t n = 0;
+    for (const auto* v : a) n += v->size();
+    bool ok = chain_model_.alloc(n) == hipSuccess;
+    size_t off = 0;
+    for (const auto* v : a) {
+        ok = ok && hipMemcpy(chain_model_.p + off, v->data(), v->size() * sizeof(double), hipMemcpyHostToDevice) == hipSuccess;
+        off += v->size();
+    }
+    if (!ok) (void)hipGetLastError();
+    chain_fresh_ = ok;
+    return ok;
+}
+
 template <typename T>
 psvfwi_status Plan<T>::get_model_gradient(int shot, double* gl, double* gm, double* gr) const
 {
     if (!gl || !gm || !gr) return fail(PSVFWI_E_ARG, "get_model_gradient: null array");
     const size_t n = (size_t)g_.nzt * g_.nxt, na = (size_t)(g_.nzt - 1) * (g_.nxt - 1);
+    if (disc_done_ && shot >= -1 && shot < nslots_ && chain_upload() && chain_out_.reserve(3 * n) == hipSuccess &&
+        chain_order_.reserve((size_t)nslots_) == hipSuccess) {
+        const std::vector<int> order = shot < 0 ? slot_of_shot_ : std::vector<int>(1, slot_of_shot_[(size_t)shot]);
+        PSV_HIP(hipMemcpy(chain_order_.p, order.data(), order.size() * sizeof(int), hipMemcpyHostToDevice));
+        const T* g[5];
+        for (int k = 0; k < 5; k++) g[k] = dg_[k].p + org_;
+        const double* m = chain_model_.p;
+        const psv::ChainModel cm{m, m + n, m + n + na, m + n + 2 * na};
+        PSV_HIP(psv::launch_chain_gradient<T>(g, fst_, chain_order_.p, (int)order.size(), g_.nzt, g_.nxt, pitch_, cm,
+                                              chain_out_.p, stream_));
+        double* out[3] = {gl, gm, gr};
+        for (int k = 0; k < 3; k++)
+            PSV_HIP(hipMemcpyAsync(out[k], chain_out_.p + k * n, n * sizeof(double), hipMemcpyDeviceToHost, stream_));
+        PSV_HIP(hipStreamSynchronize(stream_));
+        return PSVFWI_OK;
+    }
+    (void)hipGetLastError();
     std::vector<double> c0(n), c1(n), c2(na), c3(na), c4(na);
     PSV_TRY(get_coefficient_gradient(shot, c0.data(), c1.data(), c2.data(), c3.data(), c4.data()));
     return psvfwi_chain_gradient(g_.nzt, g_.nxt, h_mu_.data(), h_mu_zx_.data(), h_rho_zp_.data(),
@@ -304,6 +342,7 @@ psvfwi_status Plan<T>::get_model_gradient(int shot, double* gl, double* gm, doub
     template Plan<T>::View Plan<T>::entry(const T*, int) const; \
     template psv::DiscreteParams<T> Plan<T>::dparams(int, const View&, const View&); \
     template psvfwi_status Plan<T>::get_coefficient_gradient(int, double*, double*, double*, double*, double*) const; \
+    template bool Plan<T>::chain_upload() const; \
     template psvfwi_status Plan<T>::get_model_gradient(int, double*, double*, double*) const;
 PSV_FOR_EACH_PRECISION(PSV_INSTANTIATE)
 

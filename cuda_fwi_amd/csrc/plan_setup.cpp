@@ -99,6 +99,7 @@ psvfwi_status Plan<T>::set_model(const double* lam, const double* mu, const doub
     h_mu_.assign(mu, mu + (size_t)nzt * nxt);
     const size_t na = (size_t)(nzt - 1) * (nxt - 1);
     h_mu_zx_.assign(mu_zx, mu_zx + na);
+    chain_fresh_ = false;
     h_rho_zp_.assign(rho_zp, rho_zp + na);
     h_rho_xp_.assign(rho_xp, rho_xp + na);
     have_model_ = true;

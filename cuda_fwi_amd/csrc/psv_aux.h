@@ -17,6 +17,17 @@ template <typename T>
 hipError_t launch_grad_sum(const T* grad, size_t gst, const int* order, int nshots, size_t n,
                            double* out, hipStream_t s);
 
+// The exact gradient with respect to lam, mu, rho from the five coefficient gradients, in FP64
+// (the arithmetic of psvfwi_chain_gradient on their sums over `nshots` shots in the order
+// `order`): g[i] + order[k] * gst is a shot's array, `pitch` elements a row; the averaged
+// arrays have one row and one column less.
+struct ChainModel {
+    const double *mu, *mu_zx, *rho_zp, *rho_xp;
+};
+template <typename T>
+hipError_t launch_chain_gradient(const T* const g[5], size_t gst, const int* order, int nshots, int nzt, int nxt,
+                                 int pitch, const ChainModel& m, double* out, hipStream_t s);
+
 template <typename T>
 hipError_t launch_fill(T* p, size_t n, T v, hipStream_t s);
 
