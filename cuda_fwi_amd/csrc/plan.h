@@ -243,6 +243,14 @@ private:
         int res_gen = -1;
     };
 
+    // tiles of the resident loop: strips[k] to strips[k + 1] are the tiles of a launch; with more
+    // than one, a launch takes at most `steps` steps
+    struct Partition {
+        std::vector<psv::ResTile> h;
+        std::vector<int> strips;
+        int steps = 0;
+    };
+
     // the resident time loop (plan_resident.cpp): the tiles chosen for a batch of `slots`
     // shots (shape < 0: it does not fit), conc slots per launch
     struct Resident {
@@ -252,7 +260,8 @@ private:
         bool discrete = false;  // ... and its shape has the replay and the reverse steps
         bool uploaded = false;
         int kdiv = 0;           // some CPML K differs from 1
-        std::vector<psv::ResTile> h;
+        Partition part;
+        DBuf<T> other[psv::kStateArrays];  // more strips: a slot's state after their steps
         DBuf<psv::ResTile> tiles;
         DBuf<unsigned long long> exch;
         size_t exch_slot = 0;
@@ -296,7 +305,7 @@ private:
                                 const Tables& tab, bool fwd_sig, hipGraphExec_t* out);
 
     // ------------------------------------------------------- plan_resident.cpp
-    std::vector<psv::ResTile> resident_tiles(const psv::ResShape& sh, bool discrete, int most_rows) const;
+    Partition resident_tiles(const psv::ResShape& sh, bool discrete, int most_rows, int cap) const;
     size_t resident_terms() const;
     bool chain_upload() const;
     bool resident_ready();

@@ -11,7 +11,7 @@ namespace {
 // The rows of one column of tiles.  A tile is interior when the rows it owns are in
 // [zlo, zhi) (and xin, the same in x).  Interior tiles take up to `own` rows, edge tiles up to
 // `own_edge`; the fewest tiles that cover the column.
-void tile_column(int nzt, int zlo, int zhi, bool xin, int own, int own_edge, int x0, int x1, int xr,
+void tile_column(int nzt, int zlo, int zhi, bool xin, int own, int own_edge, int x0, int x1,
                  std::vector<psv::ResTile>& out)
 {
     // need[z]: tiles for the rows from z on; step[z]: height of the first, negative for interior
@@ -34,7 +34,7 @@ void tile_column(int nzt, int zlo, int zhi, bool xin, int own, int own_edge, int
         t.x0 = x0;
         t.x1 = x1;
         t.zr = std::max(0, z - psv::kResHalo);
-        t.xr = xr;
+        t.xr = std::max(0, x0 - psv::kResHalo);
         t.edge = step[(size_t)z] < 0 ? 0 : 1;
         out.push_back(t);
         z += h;
@@ -43,12 +43,12 @@ void tile_column(int nzt, int zlo, int zhi, bool xin, int own, int own_edge, int
 
 }  // namespace
 
-// The tiles of the grid for a shape.  Interior tiles: every stress cell they compute (2 cells
-// around the owned ones) is updated, outside the CPML strips and below the free-surface row;
-// for the transposed steps also every velocity weight they form (kResHalo cells around) is one of an
-// updated cell outside the strips, and none of their stress cells is mirrored.
+// The tiles of the grid for a shape, in strips of at most `cap` (none: they do not fit).  Interior tiles: every stress cell they compute (2 cells around the owned ones)
+// is updated, outside the CPML strips and below the free-surface row; for the transposed steps also
+// every velocity weight they form (kResHalo cells around) is one of an updated cell outside the
+// strips, and none of their stress cells is mirrored.
 template <typename T>
-std::vector<psv::ResTile> Plan<T>::resident_tiles(const psv::ResShape& sh, bool discrete, int most_rows) const
+typename Plan<T>::Partition Plan<T>::resident_tiles(const psv::ResShape& sh, bool discrete, int most_rows, int cap) const
 {
     const int nzt = g_.nzt, nxt = g_.nxt, H = fpad_;
     const bool pml = g_.npml > 0;
@@ -63,25 +63,55 @@ std::vector<psv::ResTile> Plan<T>::resident_tiles(const psv::ResShape& sh, bool 
     }
     const int own = std::min(sh.rows * sh.waves - 2 * psv::kResHalo, most_rows);
     const int own_edge = std::min(sh.rows_edge * sh.waves - 2 * psv::kResHalo, most_rows);
-    std::vector<psv::ResTile> out;
+    auto column = [&](int x0, int x1) {
+        std::vector<psv::ResTile> t;
+        tile_column(nzt, zlo, zhi, x0 >= xlo && x1 <= xhi, own, own_edge, x0, x1, t);
+        return t;
+    };
     // columns: the first and last tile have a halo on one side only
     const int W = psv::kResOwnX, end = W + psv::kResHalo;
     const int ncol = nxt <= 64 ? 1 : (nxt <= 2 * end ? 2 : 2 + (nxt - 2 * end + W - 1) / W);
+    std::vector<std::vector<psv::ResTile>> col;
     for (int c = 0, x = 0; c < ncol; c++) {
         // even widths, within what each column can hold
         const int left = ncol - 1 - c, rest = left == 0 ? 0 : (left - 1) * W + end;
         const int most = ncol == 1 ? 64 : (c == 0 || left == 0 ? end : W);
         const int x1 = x + std::min(most, std::max((nxt - x + left) / (left + 1), nxt - x - rest));
-        const bool xin = x >= xlo && x1 <= xhi;
-        tile_column(nzt, zlo, zhi, xin, own, own_edge, x, x1, std::max(0, x - psv::kResHalo), out);
+        col.push_back(column(x, x1));
         x = x1;
     }
-    int rows = 0;
-    for (psv::ResTile& t : out) {
-        t.row0 = rows;
-        rows += sh.waves * (t.edge ? sh.rows_edge : sh.rows);
-    }
-    return out;
+    // the fewest strips of even numbers of columns, then the most columns around each
+    for (int n = 1; n <= ncol; n++)
+        for (int around = n == 1 ? 1 : psv::kStripColumns; around >= 1; around--) {
+            Partition p;
+            p.strips.assign(1, 0);
+            p.steps = around * psv::kStripSteps;
+            const int ext = around * psv::kStripCells;
+            int rows = 0;
+            bool fits = true;
+            for (int k = 0; k < n && fits; k++) {
+                const int c0 = k * ncol / n, c1 = (k + 1) * ncol / n;
+                const int xa = col[(size_t)c0][0].x0, xb = col[(size_t)c1 - 1][0].x1;
+                const int xs = std::max(0, xa - ext), xe = std::min(nxt, xb + ext);
+                auto add = [&](const std::vector<psv::ResTile>& ts, int shadow) {
+                    for (psv::ResTile t : ts) {
+                        t.xs = xs;
+                        t.xe = xe;
+                        t.shadow = shadow;
+                        t.row0 = rows;
+                        if (!shadow) rows += sh.waves * (t.edge ? sh.rows_edge : sh.rows);
+                        p.h.push_back(t);
+                    }
+                };
+                for (int c = c0; c < c1; c++) add(col[(size_t)c], 0);
+                for (int x = xa; x > xs; x -= psv::kStripCells) add(column(std::max(xs, x - psv::kStripCells), x), 1);
+                for (int x = xb; x < xe; x += psv::kStripCells) add(column(x, std::min(xe, x + psv::kStripCells)), 1);
+                fits = (int)p.h.size() - p.strips.back() <= cap;
+                p.strips.push_back((int)p.h.size());
+            }
+            if (fits) return p;
+        }
+    return Partition();
 }
 
 // A split step of `n` shots in us: two launches that a small grid does not fill, then the
@@ -92,6 +122,13 @@ static double split_step_us(double cells, int esize, bool dwords)
 {
     const double floor = dwords ? 20.0 : 12.5;
     return std::max(floor, 5.0 + cells * (esize == 4 ? 19e-6 : 39e-6));
+}
+
+// What a strip's launch of some steps takes besides them, per step: the launch, ten arrays in and
+// five out.  (Half of 2484 x 884 in FP32: 20 us between the launches and 20 us of each.)
+static double strip_move_us(double cells, int esize, int steps)
+{
+    return (20.0 + cells * 15 * esize / 4e6) / steps;
 }
 
 // Whether the plan's runs can take the resident loop, and its shape for the current batch.
@@ -110,6 +147,8 @@ bool Plan<T>::resident_ready()
     }
     // every tile needs room for the mirror rows and the rim of a neighbour
     if (g_.nxt < 16 || g_.nzt < 16) return false;
+    // the exchange buffer is addressed in 32 bits
+    if ((double)(g_.nzt + 8) * (g_.nxt + 8) * 8 * sizeof(T) >= 2147483648.0) return false;
     const bool want = grad_mode_ == PSVFWI_GRADIENT_DISCRETE;
     if (res_.slots == nslots_ && res_.want == want) return res_.shape >= 0;
     res_.slots = nslots_;
@@ -121,23 +160,27 @@ bool Plan<T>::resident_ready()
         // the shots run conc at a time, rounds times over; the split step takes them together
         double best = split_step_us((double)nslots_ * g_.nzt * g_.nxt, (int)sizeof(T), std::is_same<T, psv::dfloat>::value);
         for (int i = 0; i < n; i++) {
-            const std::vector<psv::ResTile> t = resident_tiles(shapes[i], d != 0, g_.nzt);
             int cap = 1 << 30;
             for (int mode = psv::kForward; mode <= (d ? psv::kReverse : (int)psv::kAdjoint); mode++) {
                 int c = 0;
                 if (psv::resident_capacity<T>(g_.fdorder, mode, i, &c) != hipSuccess) c = 0;
                 cap = std::min(cap, c);
             }
-            if ((int)t.size() > cap) continue;
-            const int conc = std::min(nslots_, cap / (int)t.size());
-            const int rounds = (nslots_ + conc - 1) / conc;
-            const double cost = rounds * shapes[i].us;
+            const Partition p = resident_tiles(shapes[i], d != 0, g_.nzt, cap);
+            if (p.h.empty()) continue;
+            const int ns = (int)p.strips.size() - 1;
+            const int conc = ns > 1 ? 1 : std::min(nslots_, cap / (int)p.h.size());
+            // launches a step, and what starting one and moving its state adds to a step of a strip
+            const int rounds = ns > 1 ? nslots_ * ns : (nslots_ + conc - 1) / conc;
+            const double move = ns > 1 ? strip_move_us((double)g_.nzt * g_.nxt / ns, (int)sizeof(T), p.steps) : 0.0;
+            const double cost = rounds * (shapes[i].us + move);
             if (cost < best) {
                 best = cost;
                 res_.shape = i;
                 res_.conc = conc;
-                res_.discrete = d != 0;
                 res_.cap = cap;
+                res_.part = p;
+                res_.discrete = d != 0;
             }
         }
     }
@@ -147,9 +190,41 @@ bool Plan<T>::resident_ready()
     // rows to compute leave their SIMD to the others (down to 6 rows, where a shape's two rows a
     // wave are still shared evenly; 241 x 221, 190 tiles for 115, a step: compensated FP32
     // 10.4 -> 9.0 us, FP32 and FP64 3 % less)
-    for (int own = 6;; own++) {
-        res_.h = resident_tiles(shapes[res_.shape], res_.discrete, own);
-        if ((int)res_.h.size() * res_.conc <= res_.cap || own >= g_.nzt) break;
+    for (int own = 6; own < g_.nzt; own++) {
+        const Partition p = resident_tiles(shapes[res_.shape], res_.discrete, own, res_.cap / res_.conc);
+        if (!p.h.empty() && p.strips.size() == res_.part.strips.size() && p.steps == res_.part.steps) {
+            res_.part = p;
+            break;
+        }
+    }
+    // the exchange buffer, the flag, and for strips the other set of a slot's state
+    {
+        res_.xpitch = (int)round_up((size_t)g_.nxt, 8);
+        res_.zpitch = (int)round_up((size_t)g_.nzt, 8);
+        res_.exch_slot = 2 * ((size_t)g_.nzt * res_.xpitch + (size_t)g_.nxt * res_.zpitch) * (2 * sizeof(T) / 4);
+        const size_t need = res_.exch_slot * (size_t)res_.conc;
+        bool ok = true;
+        if (!res_.exch.p || res_.exch.cap < need) {
+            ok = res_.exch.alloc(need) == hipSuccess &&
+                 psv::launch_fill<unsigned long long>(res_.exch.p, need, 0ull, stream_) == hipSuccess;
+            res_.tag = 1;
+        }
+        if (ok && !res_.aborted) {
+            ok = hipHostMalloc(reinterpret_cast<void**>(&res_.aborted), sizeof(int), hipHostMallocMapped) == hipSuccess;
+            if (ok) *res_.aborted = 0;
+        }
+        const bool two = res_.part.strips.size() > 2;
+        for (int k = 0; k < psv::kStateArrays && ok && two; k++) {
+            const size_t n = k < 5 ? fst_ : (g_.npml > 0 ? (k < 9 ? xst_ : zst_) : 0);
+            ok = res_.other[k].alloc(n) == hipSuccess && (n == 0 || psv::launch_fill<T>(res_.other[k].p, n, (T)0, stream_) == hipSuccess);
+        }
+        if (!ok) {
+            (void)hipGetLastError();
+            for (DBuf<T>& b : res_.other) b.release();
+            res_.exch.release();
+            res_.shape = -1;
+            return false;
+        }
     }
     res_.waves = shapes[res_.shape].waves;
     res_.rows = shapes[res_.shape].rows;
@@ -164,7 +239,7 @@ template <typename T>
 psvfwi_status Plan<T>::resident_points(Tables& t)
 {
     if (t.res_gen == res_.gen) return PSVFWI_OK;
-    const int ntile = (int)res_.h.size();
+    const int ntile = (int)res_.part.h.size();
     const int nw = res_.waves;
     struct Layer {
         int head;
@@ -174,7 +249,7 @@ psvfwi_status Plan<T>::resident_points(Tables& t)
     // entry `v` of component `comp` at (z, x): the first layer of its wave, row and component
     // whose lane is free, so that entries of one cell keep their order
     auto add = [&](int slot, int k, int z, int x, int comp, int rec, int v) {
-        const psv::ResTile& q = res_.h[(size_t)k];
+        const psv::ResTile& q = res_.part.h[(size_t)k];
         const int R = q.edge ? res_.rows_edge : res_.rows;
         const int row = z - q.zr, lane = x - q.xr;
         std::vector<Layer>& l = lay[((size_t)slot * ntile + k) * nw + (size_t)(row / R)];
@@ -194,10 +269,11 @@ psvfwi_status Plan<T>::resident_points(Tables& t)
                 const int* e = rec ? &t.zxc_h[3 * (size_t)g] : &t.grp_h[5 * (size_t)g];
                 const int z = e[0], x = e[1], comp = e[2];
                 for (int k = 0; k < ntile; k++) {
-                    const psv::ResTile& q = res_.h[(size_t)k];
+                    const psv::ResTile& q = res_.part.h[(size_t)k];
                     // stress sources act on the stresses a tile computes around its own cells too
                     const int ring = !rec && comp == 4 ? 2 : 0;
                     if (z < q.z0 - ring || z >= q.z1 + ring || x < q.x0 - ring || x >= q.x1 + ring) continue;
+                    if (rec && q.shadow) continue;
                     if (rec) add(s, k, z, x, comp, 1, g - off[(size_t)s]);
                     else
                         for (int j = 0; j < e[4]; j++) add(s, k, z, x, comp, 0, t.row_h[(size_t)(e[3] + j)]);
@@ -224,27 +300,14 @@ psvfwi_status Plan<T>::resident_points(Tables& t)
     return PSVFWI_OK;
 }
 
-// tiles, exchange buffer and flag of the resident loop
+// the tiles of the resident loop, on the device
 template <typename T>
 psvfwi_status Plan<T>::resident_prepare()
 {
     if (!res_.uploaded) {
-        PSV_HIP(res_.tiles.alloc(res_.h.size()));
-        PSV_HIP(hipMemcpy(res_.tiles.p, res_.h.data(), res_.h.size() * sizeof(psv::ResTile), hipMemcpyHostToDevice));
+        PSV_HIP(res_.tiles.alloc(res_.part.h.size()));
+        PSV_HIP(hipMemcpy(res_.tiles.p, res_.part.h.data(), res_.part.h.size() * sizeof(psv::ResTile), hipMemcpyHostToDevice));
         res_.uploaded = true;
-    }
-    res_.xpitch = (int)round_up((size_t)g_.nxt, 8);
-    res_.zpitch = (int)round_up((size_t)g_.nzt, 8);
-    res_.exch_slot = 2 * ((size_t)g_.nzt * res_.xpitch + (size_t)g_.nxt * res_.zpitch) * (2 * sizeof(T) / 4);
-    const size_t need = res_.exch_slot * (size_t)res_.conc;
-    if (!res_.exch.p || res_.exch.cap < need) {
-        PSV_HIP(res_.exch.alloc(need));
-        PSV_HIP(psv::launch_fill<unsigned long long>(res_.exch.p, res_.exch.cap, 0ull, stream_));
-        res_.tag = 1;
-    }
-    if (!res_.aborted) {
-        PSV_HIP(hipHostMalloc(reinterpret_cast<void**>(&res_.aborted), sizeof(int), hipHostMallocMapped));
-        *res_.aborted = 0;
     }
     return PSVFWI_OK;
 }
@@ -257,27 +320,18 @@ psvfwi_status Plan<T>::launch_resident(State<T>& st, Tables& tab, bool fwd_sig, 
 {
     PSV_TRY(resident_points(tab));
     const int steps = it1 - it0;
-    if (res_.tag > 0xffffffffu - (unsigned)steps - 2u) {
-        PSV_HIP(psv::launch_fill<unsigned long long>(res_.exch.p, res_.exch.cap, 0ull, stream_));
-        res_.tag = 1;
-    }
     psv::ResidentParams<T> a{};
     if (mode >= psv::kReplay) {
         a.terms = seg_.p;
         a.terms_slot = resident_terms();
         a.terms_step = a.terms_slot * (size_t)res_.conc;
+        a.terms_it0 = it0;
         for (int i = 0; i < 5; i++) a.g5[i] = atw(dg_[i], fst_);
     }
     a.p = base_params(st, tab, fwd_sig);
     a.p.nslots = active(it0);
     a.p.flags = flags;
     a.p.tf0 = tf0;
-    a.tiles = res_.tiles.p;
-    a.ntile = (int)res_.h.size();
-    a.it0 = it0;
-    a.it1 = it1;
-    const size_t per = (size_t)a.ntile * res_.waves;
-    a.pts.off = tab.res_off.p + (size_t)w0_ * per;
     a.pts.head = tab.res_head.p;
     a.pts.id = tab.res_id.p;
     a.tf_stride = one_plane ? 0 : (size_t)5 * nfz_ * nfx_;
@@ -285,13 +339,51 @@ psvfwi_status Plan<T>::launch_resident(State<T>& st, Tables& tab, bool fwd_sig, 
     a.exch_slot = res_.exch_slot;
     a.xpitch = res_.xpitch;
     a.zpitch = res_.zpitch;
-    a.tag = res_.tag;
     a.aborted = res_.aborted;
     a.kdiv = res_.kdiv;
-    res_.tag += (unsigned)steps;
+    T** const in[psv::kStateArrays] = {&a.p.vx, &a.p.vz, &a.p.sxx, &a.p.szx, &a.p.szz, &a.p.mvxx, &a.p.mvzx,
+                                       &a.p.msxxx, &a.p.mszxx, &a.p.mvzz, &a.p.mvxz, &a.p.mszzz, &a.p.mszxz};
+    const int nstrip = (int)res_.part.strips.size() - 1;
+    for (int k = 0; k < psv::kStateArrays; k++) a.out[k] = nstrip > 1 ? res_.other[k].p + (k < 5 ? org_ : 0) : *in[k];
     const bool sample = kind >= 0 && sample_ev_[0][0] && nsamp_ < kMaxSamples;
     if (sample) PSV_HIP(hipEventRecord(sample_ev_[nsamp_][0], stream_));
-    const hipError_t e = psv::launch_resident<T>(a, g_.fdorder, mode, res_.shape, stream_);
+    // one launch of all steps; strips (one slot at a time): an even number of launches of a few
+    // steps each, which ends in the slot's own arrays, each writing the other set of the state
+    const int last = nstrip > 1 ? std::min(it1, group_nt()) : it1, n = last - it0;
+    int parts = 1;
+    if (nstrip > 1) {
+        parts = (n + res_.part.steps - 1) / res_.part.steps;
+        parts += n > 1 ? parts & 1 : 0;
+    }
+    hipError_t e = hipSuccess;
+    for (int j = 0; j < parts && e == hipSuccess; j++) {
+        const bool back = mode == psv::kAdjoint || mode == psv::kReverse;
+        const int b0 = (int)((long long)n * j / parts), b1 = (int)((long long)n * (j + 1) / parts);
+        a.it0 = back ? last - b1 : it0 + b0;
+        a.it1 = back ? last - b0 : it0 + b1;
+        if (nstrip == 1) a.it1 = it1;
+        const unsigned span = (unsigned)(a.it1 - a.it0);
+        for (int k = 0; k < nstrip && e == hipSuccess; k++) {
+            if (res_.tag > 0xffffffffu - span - 2u) {
+                PSV_HIP(psv::launch_fill<unsigned long long>(res_.exch.p, res_.exch.cap, 0ull, stream_));
+                res_.tag = 1;
+            }
+            const int t0 = res_.part.strips[(size_t)k];
+            a.tiles = res_.tiles.p + t0;
+            a.ntile = res_.part.strips[(size_t)k + 1] - t0;
+            a.pts.off = tab.res_off.p + ((size_t)w0_ * res_.part.h.size() + (size_t)t0) * res_.waves;
+            a.tag = res_.tag;
+            res_.tag += span;
+            e = psv::launch_resident<T>(a, g_.fdorder, mode, res_.shape, stream_);
+        }
+        if (nstrip > 1)
+            for (int k = 0; k < psv::kStateArrays; k++) std::swap(*in[k], a.out[k]);
+    }
+    // (a single step ends in the other set)
+    for (int k = 0; nstrip > 1 && (parts & 1) && k < psv::kStateArrays && e == hipSuccess; k++)
+        if (res_.other[k].n > 0)
+            e = hipMemcpyAsync(a.out[k] - (k < 5 ? org_ : 0), res_.other[k].p, res_.other[k].n * sizeof(T),
+                               hipMemcpyDeviceToDevice, stream_);
     if (e != hipSuccess) {
         // refused (no cooperative launch here): the caller runs the split step instead
         (void)hipGetLastError();
@@ -313,8 +405,10 @@ psvfwi_status Plan<T>::launch_resident(State<T>& st, Tables& tab, bool fwd_sig, 
 template <typename T>
 size_t Plan<T>::resident_terms() const
 {
-    const psv::ResTile& t = res_.h.back();
-    return (size_t)(t.row0 + res_.waves * (t.edge ? res_.rows_edge : res_.rows)) * 320;
+    size_t rows = 0;
+    for (const psv::ResTile& t : res_.part.h)
+        if (!t.shadow) rows = std::max(rows, (size_t)t.row0 + res_.waves * (t.edge ? res_.rows_edge : res_.rows));
+    return rows * 320;
 }
 
 // After the stream has drained: a resident run whose waits ran out, or that was refused,
@@ -329,7 +423,7 @@ bool Plan<T>::resident_failed()
 }
 
 #define PSV_INSTANTIATE(T) \
-    template std::vector<psv::ResTile> Plan<T>::resident_tiles(const psv::ResShape&, bool, int) const; \
+    template Plan<T>::Partition Plan<T>::resident_tiles(const psv::ResShape&, bool, int, int) const; \
     template bool Plan<T>::resident_ready(); \
     template size_t Plan<T>::resident_terms() const; \
     template psvfwi_status Plan<T>::resident_points(Tables&); \

@@ -19,9 +19,24 @@ constexpr int kResOwnX = 64 - 2 * kResHalo;    // columns a tile owns between tw
 struct ResTile {
     int z0, z1, x0, x1;
     int zr, xr;
-    int edge;  // the region meets a CPML strip, the free surface or the grid's frame
-    int row0;  // rows of all waves of the tiles before this one
+    int edge;    // the region meets a CPML strip, the free surface or the grid's frame
+    int row0;    // rows of all waves of the tiles before this one
+    int xs, xe;  // columns of the launch: it has no tiles outside
+    int shadow;  // computed for its neighbours only, writes nothing
+    int pad;
 };
+
+// A grid with more tiles than CUs runs as strips of columns, some steps at a time: without
+// neighbours the outer kResHalo columns of a strip go wrong every step, so a strip has more columns
+// of tiles on each side that are computed and thrown away, each kStripCells wide, which lasts for
+// kStripSteps steps.
+constexpr int kStripSteps = kResOwnX / kResHalo;
+constexpr int kStripCells = kStripSteps * kResHalo;
+constexpr int kStripColumns = 4;  // at most
+
+// The state's arrays in the order vx, vz, sxx, szx, szz, mvxx, mvzx, msxxx, mszxx, mvzz, mvxz,
+// mszzz, mszxz.
+constexpr int kStateArrays = 13;
 
 // Point sources and receivers of a (slot, tile, wave): layers of at most one entry per
 // lane, in the order they act; head: row | comp << 8 | receiver << 16; id: signal row or
@@ -53,10 +68,13 @@ struct ResidentParams {
     unsigned tag;            // tag of the launch's first step
     int* aborted;            // host memory: set when a wait ran out
     int kdiv;                // some CPML K differs from 1
+    T* out[kStateArrays];    // the state after the steps: p's own arrays, or another set where
+                             // strips still have to read the state before them
     // replay and reverse: five values per cell, [step - it0][slot][row of a wave][5][64 lanes],
     // and the reverse steps' gradients (lam, mu, mu_zx, rho_zp, rho_xp)
-    T* terms;
+    T* terms;                // (of step terms_it0)
     size_t terms_step, terms_slot;
+    int terms_it0;
     T* g5[5];
 };
 

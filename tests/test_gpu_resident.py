@@ -3,7 +3,7 @@ wavefields in registers, tiles that exchange their rims) against the split step 
 the oracle's tests pin: records, wavefields, CPML memory, illumination and both gradients, bit
 for bit, at the sizes where a tile can go wrong: the smallest grid, one tile to three columns of
 them, every tile shape of the three types, both orders, the free surface, no CPML, K != 1,
-checkpoint segments with a short last one, uneven shots, sources of every kind, a strided window."""
+checkpoint segments with a short last one, grids in strips, uneven shots, sources of every kind, a strided window."""
 import numpy as np
 import pytest
 
@@ -32,6 +32,8 @@ CASES = [
     (760, 520, 30, 2, 1, "fp32", 40, 1.0),
     (1000, 500, 40, 4, 0, "fp32", 40, 1.0),
     (1400, 600, 40, 4, 1, "fp32", 24, 1.0),
+    (1900, 700, 20, 4, 1, "fp32", 45, 1.5),    # strips; the last segment is one step
+    (1000, 600, 20, 2, 0, "fp64", 45, 1.0),
 ]
 
 
@@ -62,7 +64,7 @@ def _same(x, y):
 def test_resident_equals_split_step(case):
     print(f"resident {case}", flush=True)
     nt, prec = case[6], case[5]
-    for comp, window, mode in ((2, dict(dt=2), ("full", 0)), (4, dict(dt=3, dx=2, dz=3), ("checkpoint", nt // 2 - 1))):
+    for comp, window, mode in ((2, dict(dt=2), ("full", 0)), (4, dict(dt=3, dx=2, dz=3), ("checkpoint", (nt - 1) // 2))):
         pb, shots, obs = _problem(case, comp, window)
         out = []
         for tz in (8, None):
