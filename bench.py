@@ -35,6 +35,9 @@ KERNEL_NAMES = {"forward_stress": "psv_stress_kernel (forward)",
                 "forward_velocity": "psv_velocity_kernel (forward)",
                 "adjoint_stress": "psv_stress_kernel (adjoint: displacement + gradient correlation)",
                 "adjoint_velocity": "psv_velocity_kernel (adjoint)"}
+# the resident time loop: one kernel for many steps; its launches are counted in steps
+RESIDENT_NAMES = {"forward_stress": "psv_resident_kernel (forward, per step)",
+                  "adjoint_stress": "psv_resident_kernel (adjoint: displacement + gradient correlation, per step)"}
 HBM_PEAK_GBS = 8000.0
 
 
@@ -115,6 +118,21 @@ def alg_bytes(w, nwin, fwi_dt, esize):
         "adjoint_stress": s * (52 * n + 16 * strip + 44 * nwin / fwi_dt),
         "adjoint_velocity": s * (24 * n + 16 * strip),
     }
+
+
+def resident_bytes(nwin, fwi_dt, esize):
+    """HBM bytes a step of the resident time loop has to move: the state, the model and the CPML
+    memory stay in registers, so only the 20 B per window cell and stored or correlated step
+    (amortised over fwi_dt) are left.  Keys as in alg_bytes."""
+    b = 20 * nwin / fwi_dt * esize / 4.0
+    return {"forward_stress": b, "forward_velocity": 0.0, "adjoint_stress": b, "adjoint_velocity": 0.0}
+
+
+def step_kernel_name(plan_tile, resident):
+    if resident:
+        return "resident time loop (many steps per launch)"
+    return ("split (stress, velocity)" if plan_tile > 0 else
+            "fused tile" if plan_tile > -32 else "z-marching segments")
 
 
 def cpu_baseline(w, window, nt_sample, threaded=False):
@@ -228,6 +246,9 @@ def run_c2(args):
     # of a step in the ratio of their sampled event-bracketed durations (a
     # single bracketed kernel also carries the event's own dispatch overhead).
     sampled = {k: sum(u * n for u, n in v) / max(sum(n for _, n in v), 1) for k, v in ksum.items()}
+    resident = sampled["forward_velocity"] == 0 and sampled["adjoint_velocity"] == 0
+    if resident:
+        kb_all = resident_bytes(nwin, fwi_dt, esize)
     kus = {}
     for kind, ms, n in (("forward", tf_ms, nf), ("adjoint", ta_ms, na)):
         step_us = ms * 1e3 / n
@@ -242,7 +263,7 @@ def run_c2(args):
     achieved = kb / per_launch_s / 1e9
     traffic = None
     prof = os.path.join(ROOT, "profiles", "pmc_traffic_c2.json")
-    if os.path.exists(prof):
+    if os.path.exists(prof) and not resident:
         traffic = json.load(open(prof)).get(kname)
     cells = w.interior_cells()
     value = 2.0 * cells * w.nt * args.steps / T / 1e9
@@ -261,10 +282,11 @@ def run_c2(args):
                                           args.store, f"checkpoint every {args.interval}"),
                    "fwi_time_decimation": fwi_dt,
                    "tile": [64, abs(plan.tile)],
-                   "step_kernel": "fused (one launch per step)" if plan.tile < 0 else "split (stress, velocity)",
+                   "step_kernel": step_kernel_name(plan.tile, resident),
                    "tile_choice": "autotuned" if args.tile == 0 else "fixed",
                    "graph_steps": args.graph_steps},
-        "roofline": {"bound": "hbm", "kernel": KERNEL_NAMES[kname],
+        "roofline": {"bound": "rim exchange and instructions" if resident else "hbm",
+                     "kernel": (RESIDENT_NAMES if resident else KERNEL_NAMES)[kname],
                      "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
                      "alg_bytes_per_launch": int(kb), "avg_launch_us": round(kus[kname], 2),
@@ -532,7 +554,8 @@ def run_c4(args):
     # kernel, tile, shot order and launch group tuned once on the first (longest) group
     plan.set_shots([descs[i] for i in groups[0]])
     tile = args.tile if args.tile != 0 else plan.autotune(min(args.tune_steps, w.nt))
-    plan.set_tile(tile)
+    if args.tile:
+        plan.set_tile(tile)
     if args.shot_order >= 0:
         plan.set_shot_order(args.shot_order)
     band = plan.shot_order()
@@ -547,7 +570,6 @@ def run_c4(args):
         """One step: the group's fwd + misfit + adj + gradient; returns loop ms, launches and
         sampled kernel us of the forward and the adjoint."""
         plan.set_shots([descs[i] for i in g])
-        plan.set_tile(tile)
         plan.set_shot_order(band)
         plan.set_observed([obs[i] for i in g])
         plan.forward(energy=False, gradient=True)
@@ -599,6 +621,12 @@ def run_c4(args):
     # HIP events on the plan's stream, averaged over the samples of all timed steps
     direct = {k: sum(v * n for v, n in samples[k]) / max(sum(n for _, n in samples[k]), 1) for k in kinds}
     nsamp = {k: sum(n for _, n in samples[k]) for k in kinds}
+    resident = direct["forward_velocity"] == 0 and direct["adjoint_velocity"] == 0
+    streamed_total = sum(alg_kernel.values())  # what a step that streams its state would move
+    if resident:
+        rb = resident_bytes(nwin, fwi_dt, esize)
+        alg_kernel = {k: alg_kernel[k] * rb[k] / kb[k] for k in kinds}
+        kb = rb
     kus_total = {}
     for kind in ("forward", "adjoint"):
         a = direct[kind + "_stress"]
@@ -615,7 +643,7 @@ def run_c4(args):
     # from a separate rocprofv3 run), times the shots per launch of this run
     traffic = None
     prof = os.path.join(ROOT, "profiles", "pmc_traffic_c4.json")
-    if os.path.exists(prof) and esize == 4:
+    if os.path.exists(prof) and esize == 4 and not resident:
         k = json.load(open(prof))["kernels"].get(kname)
         if k:
             traffic = int(k["traffic_bytes_per_shot_step"] * bytes_per_launch / kb[kname])
@@ -628,7 +656,8 @@ def run_c4(args):
     p1 = new_plan()
     p1.set_model(lam, mu, *avg0)
     p1.set_shots([descs[0]])
-    p1.set_tile(tile)
+    if args.tile:
+        p1.set_tile(tile)
     p1.set_observed([obs[0]])
     p1.forward(energy=False, gradient=True)   # warm-up
     p1.misfit()
@@ -640,7 +669,6 @@ def run_c4(args):
     per_cells = 0
     for i in per:
         p1.set_shots([descs[i]])
-        p1.set_tile(tile)
         p1.set_observed([obs[i]])
         p1.forward(energy=False, gradient=True)
         p1.misfit()
@@ -669,11 +697,11 @@ def run_c4(args):
                                       f"{args.store_budget_gb} GB of store" if args.store == "full" else
                                       f"checkpoint every {args.interval} steps, segments recomputed "
                                       "(recomputation not counted)"),
-                   "tile": tile, "step_kernel": ("split (stress, velocity)" if tile > 0 else
-                                                 "fused tile" if tile > -32 else "z-marching segments"),
+                   "tile": tile, "step_kernel": step_kernel_name(tile, resident),
                    "shot_order": "shot-major" if band == 0 else f"bands of {band} tile rows",
                    "launch_group": lgroup or "whole group", "graph_steps": args.graph_steps},
-        "roofline": {"bound": "hbm", "kernel": KERNEL_NAMES[kname], "achieved": round(achieved, 1),
+        "roofline": {"bound": "rim exchange and instructions" if resident else "hbm",
+                     "kernel": (RESIDENT_NAMES if resident else KERNEL_NAMES)[kname], "achieved": round(achieved, 1),
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                      "traffic": traffic,
                      "traffic_source": ("stored profile, not measured in this run: rocprofv3 FETCH_SIZE + "
@@ -691,12 +719,14 @@ def run_c4(args):
                                       "sampled_us_per_launch: the event-bracketed durations of every 64th "
                                       "launch, each with one event's overhead"},
         "hbm": {"alg_bytes": int(alg_total), "alg_GBps": round(alg_total / T / 1e9, 1),
+                "streaming_step_GBps": round(streamed_total / T / 1e9, 1),
                 "frac_of_peak": round(alg_total / T / 1e9 / HBM_PEAK_GBS, 4),
                 "in_time_loops": round((loop_ms["forward"] + loop_ms["adjoint"]) / 1e3 / T, 4),
                 "frac_of_peak_in_time_loops": round(alg_total / ((loop_ms["forward"] + loop_ms["adjoint"]) / 1e3)
                                                     / 1e9 / HBM_PEAK_GBS, 4),
-                "note": "algorithmic bytes of forward + adjoint + gradient of every timed step over the "
-                        "wall time of the timed steps; in_time_loops: the share of that wall time inside "
+                "note": "algorithmic bytes of forward + adjoint + gradient of every timed step (of the "
+                        "resident loop: the stored states; streaming_step_GBps counts those of a step "
+                        "that streams its state) over the wall time of the timed steps; in_time_loops: the share of that wall time inside "
                         "the forward and adjoint time loops (HIP events), the rest being shot tables, "
                         "observed-trace uploads and the misfit"},
         "batched_shots_per_s": round(batched_rate, 3),
@@ -726,7 +756,8 @@ def c4_extras(args, line):
         plan.set_window(window)
         plan.set_model(lam, mu, *P.average_parameters(mu, rho))
         plan.set_shots(_shot_descs(w, g))
-        plan.set_tile(min(abs(line["config"]["tile"]), 16) if line["config"]["tile"] > 0 else 8)
+        if args.tile:
+            plan.set_tile(min(abs(args.tile), 16) if args.tile > 0 else 8)
         plan.set_observed([np.zeros((len(w.shots[i]["rec"]["x"]), w.shots[i]["nt"])) for i in g])
         _sync()
         t0 = time.perf_counter()

@@ -135,13 +135,20 @@ psvfwi_status psvfwi_set_shots(psvfwi_plan* plan, int nshots, const psvfwi_shot_
  * state, stress ring recomputed); tz = -32 or -64: one launch per step in
  * which each workgroup marches down a segment of 64 columns x |tz| rows,
  * every stress row computed once (ping-pong state), plus a small launch for
- * the point sources and receivers; 0 = default (8).  Every choice gives the
- * same results bit for bit. */
+ * the point sources and receivers; 0 = default: the resident time loop (many
+ * steps in one launch, the wavefields in registers) where the precision, the
+ * CPML profiles, the grid and the batch allow it and it is expected to be
+ * faster, else two launches on tiles of 8 rows.  Random-boundary and
+ * snapshot runs, and checkpoints less than 8 steps apart, take the two
+ * launches.  Every choice gives the same results bit for bit. */
 psvfwi_status psvfwi_set_tile(psvfwi_plan* plan, int tz);
 
-/* Autotuner: times `steps` forward steps of the current batch with every
+/* Autotuner: times `steps` forward steps of the current batch with the
+ * resident time loop (over up to four times the steps) and with every
  * step kernel and tile height of psvfwi_set_tile, keeps the fastest and
- * returns its psvfwi_set_tile value in *best_tile (may be NULL); for a batch it
+ * returns its psvfwi_set_tile value in *best_tile (may be NULL; 8 where the
+ * resident loop was the fastest, which psvfwi_set_tile(plan, 0) asks for and
+ * psvfwi_set_tile(plan, 8) rules out); for a batch it
  * then chooses the shot order (psvfwi_set_shot_order) and, with the split
  * step, the launch group (psvfwi_set_launch_group) the same way.  In the
  * random-boundary store mode only the split kernels (tz > 0) are tried.
@@ -153,7 +160,8 @@ psvfwi_status psvfwi_autotune(psvfwi_plan* plan, int steps, int* best_tile);
 /* Order of the workgroups of a batched launch (no counterpart in the reference, which runs
  * one shot per launch): band 0 = shot-major (every tile of shot 0, then shot 1, ...); band
  * k > 0 = bands of k tile rows, and within a band the shots one after another.  psvfwi_autotune
- * chooses among 0, 1 and 4 for batches of more than one shot.  Results do not depend on it. */
+ * chooses among 0, 1 and 4 for batches of more than one shot.  Results do not depend on it.
+ * (The resident time loop has no such order.) */
 psvfwi_status psvfwi_set_shot_order(psvfwi_plan* plan, int band);
 psvfwi_status psvfwi_get_shot_order(const psvfwi_plan* plan, int* band);
 
@@ -162,7 +170,7 @@ psvfwi_status psvfwi_get_shot_order(const psvfwi_plan* plan, int* band);
  * before the next (slots are the shots sorted by decreasing nt), so that a group's
  * wavefields stay in the GPU's 256 MB Infinity Cache from one step to the next; 0 (default)
  * steps the whole batch together.  The fused step (tile < 0) always runs the batch as one
- * group.  psvfwi_autotune chooses among 0, 16, 12, 8, 6, 4 and 2 for batches.  Results do not
+ * group, the resident time loop as many shots as fit in the registers.  psvfwi_autotune chooses among 0, 16, 12, 8, 6, 4 and 2 for batches.  Results do not
  * depend on it. */
 psvfwi_status psvfwi_set_launch_group(psvfwi_plan* plan, int shots);
 psvfwi_status psvfwi_get_launch_group(const psvfwi_plan* plan, int* shots);
@@ -170,8 +178,8 @@ psvfwi_status psvfwi_get_launch_group(const psvfwi_plan* plan, int* shots);
 /* Graph-captured time loop: with steps > 0 (even), forward and adjoint
  * runs replay HIP graphs of `steps` consecutive step launches (the step index
  * is read from device memory) over every run of steps in which the set of
- * active shots does not change; checkpointed stores and snapshots keep the
- * direct launches.  0 (default) launches every step directly.  Results are
+ * active shots does not change; checkpointed stores, snapshots and the
+ * resident time loop keep the direct launches.  0 (default) launches every step directly.  Results are
  * identical either way; per-kernel timing samples are taken only from direct
  * launches.  (No counterpart in the reference, which launches two kernels per
  * step and synchronizes after each, CUDA_week2/forward_kernel_PSV_GPU.cu:585-600.) */
@@ -269,13 +277,14 @@ psvfwi_status psvfwi_chain_gradient(int nzt, int nxt, const double* mu, const do
                                     double* out_rho);
 
 /* Timing of the last forward/adjoint call (milliseconds, HIP events) and the
- * number of step-kernel launches it made. */
+ * number of step-kernel launches it made (the resident time loop: steps). */
 psvfwi_status psvfwi_last_timing(const psvfwi_plan* plan, double* ms, long* launches);
 
 /* Per-kernel durations sampled (HIP events on the plan's stream, every 64th
  * step) during the last forward / adjoint call: kind 0 forward steps, 1
  * adjoint steps, 2 checkpoint replay steps; mean microseconds of the stress
- * kernel and of the velocity kernel, and the number of samples.  (A
+ * kernel and of the velocity kernel, and the number of samples.  The resident
+ * time loop has one kernel: its launches' time per step, and 0.  (A
  * measurement hook with no counterpart in the reference, which only prints
  * clock() totals, CUDA_week2/fd_wave_model.cu:593-595.) */
 psvfwi_status psvfwi_kernel_timing(const psvfwi_plan* plan, int kind, double* us_stress,
