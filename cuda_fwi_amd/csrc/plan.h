@@ -86,6 +86,7 @@ struct psvfwi_plan {
     virtual psvfwi_status get_model_gradient(int, double*, double*, double*) const = 0;
     virtual psvfwi_status timing(double*, long*) const = 0;
     virtual psvfwi_status kernel_timing(int, double*, double*, int*) const = 0;
+    virtual psvfwi_status last_step(int, int*, int*) const = 0;
 };
 
 namespace psvplan {
@@ -200,6 +201,7 @@ public:
     psvfwi_status autotune(int steps, int* best) override;
     psvfwi_status timing(double* ms, long* launches) const override;
     psvfwi_status kernel_timing(int kind, double* us_stress, double* us_velocity, int* samples) const override;
+    psvfwi_status last_step(int kind, int* tile, int* gave_up) const override;
 
     // -------------------------------------------------------- plan_forward.cpp
     psvfwi_status forward(int flags) override;
@@ -528,6 +530,14 @@ private:
     static constexpr int kMaxSamples = 512;
     double last_ms_ = 0;
     long launches_ = 0;
+    // what the last forward (0) and adjoint (1) ran on: 0 the resident loop, else the tile
+    bool ran_step_[2] = {};
+    int ran_tile_[2] = {};
+    void ran_on(int kind, bool resident)
+    {
+        ran_step_[kind] = true;
+        ran_tile_[kind] = resident ? 0 : tz_;
+    }
     static constexpr int kNumCand = 8;
     float tune_ms_[kNumCand] = {};
     hipEvent_t sample_ev_[kMaxSamples][3] = {};

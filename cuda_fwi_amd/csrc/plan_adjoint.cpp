@@ -168,6 +168,7 @@ psvfwi_status Plan<T>::adjoint(int flags)
     PSV_HIP(hipEventElapsedTime(&ms, ev0_, ev1_));
     last_ms_ = ms;
     PSV_TRY(collect_samples());
+    ran_on(1, resident);
     ran_ = true;
     adj_grad_done_ = grad;
     parity_ = false;  // every shot ends at it = 0
@@ -273,6 +274,7 @@ psvfwi_status Plan<T>::adjoint_rb(int flags)
     PSV_HIP(hipEventElapsedTime(&ms, ev0_, ev1_));
     last_ms_ = ms;
     PSV_TRY(collect_samples());
+    ran_on(1, false);
     ran_ = true;
     adj_grad_done_ = true;
     fwd_grad_done_ = false;  // the forward's final state has been consumed

@@ -153,6 +153,7 @@ psvfwi_status Plan<T>::adjoint_discrete()
     float ms = 0;
     PSV_HIP(hipEventElapsedTime(&ms, ev0_, ev1_));
     last_ms_ = ms;
+    ran_on(1, resident);
     adj_grad_done_ = false;
     disc_done_ = true;
     return PSVFWI_OK;

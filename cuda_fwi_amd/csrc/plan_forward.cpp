@@ -111,6 +111,7 @@ psvfwi_status Plan<T>::forward(int flags)
     PSV_HIP(hipEventElapsedTime(&ms, ev0_, ev1_));
     last_ms_ = ms;
     PSV_TRY(collect_samples());
+    ran_on(0, resident);
     ran_ = true;
     fwd_done_ = true;
     fwd_grad_done_ = grad;

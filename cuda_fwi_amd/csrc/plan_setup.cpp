@@ -170,6 +170,7 @@ psvfwi_status Plan<T>::set_tile(int tz)
                                   "-32 or -64 (z-marching step)");
     tz_ = tz;
     tile_auto_ = !chosen;
+    if (tile_auto_) res_.failed = false;  // asked for again
     return PSVFWI_OK;
 }
 

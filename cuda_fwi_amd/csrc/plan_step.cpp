@@ -384,7 +384,18 @@ psvfwi_status Plan<T>::kernel_timing(int kind, double* us_stress, double* us_vel
     return PSVFWI_OK;
 }
 
+template <typename T>
+psvfwi_status Plan<T>::last_step(int kind, int* tile, int* gave_up) const
+{
+    if (kind < 0 || kind > 1) return fail(PSVFWI_E_ARG, "last_step: kind must be 0 or 1");
+    if (!ran_step_[kind]) return fail(PSVFWI_E_STATE, "last_step: no such run yet");
+    if (tile) *tile = ran_tile_[kind];
+    if (gave_up) *gave_up = res_.failed;
+    return PSVFWI_OK;
+}
+
 #define PSV_INSTANTIATE(T) \
+    template psvfwi_status Plan<T>::last_step(int, int*, int*) const; \
     template psvfwi_status Plan<T>::autotune(int, int*); \
     template psvfwi_status Plan<T>::timing(double*, long*) const; \
     template psvfwi_status Plan<T>::capture_steps(psv::StepParams<T>, int, int, State<T>&, State<T>&, const Tables&, bool, hipGraphExec_t*); \

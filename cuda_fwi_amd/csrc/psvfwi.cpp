@@ -329,6 +329,12 @@ psvfwi_status psvfwi_kernel_timing(const psvfwi_plan* plan, int kind, double* us
     return plan->kernel_timing(kind, us_stress, us_velocity, samples);
 }
 
+psvfwi_status psvfwi_last_step(const psvfwi_plan* plan, int kind, int* tile, int* gave_up)
+{
+    PSV_PLAN(plan);
+    return plan->last_step(kind, tile, gave_up);
+}
+
 psvfwi_status psvfwi_parabola_step(const double* L2, const double* step, double* opt)
 {
     if (!L2 || !step || !opt) return fail(PSVFWI_E_ARG, "parabola_step: null argument");

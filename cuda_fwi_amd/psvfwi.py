@@ -39,7 +39,7 @@ EXPORTS = ("psvfwi_last_error", "psvfwi_plan_create", "psvfwi_plan_destroy", "ps
            "psvfwi_set_gradient_mode", "psvfwi_get_coefficient_gradient", "psvfwi_get_model_gradient",
            "psvfwi_chain_gradient", "psvfwi_random_boundary", "psvfwi_set_shot_order",
            "psvfwi_get_shot_order", "psvfwi_set_launch_group", "psvfwi_get_launch_group",
-           "psvfwi_misfit_noalloc")
+           "psvfwi_misfit_noalloc", "psvfwi_last_step")
 
 
 class PsvfwiError(RuntimeError):
@@ -341,6 +341,13 @@ class Plan:
         a, b, n = C.c_double(), C.c_double(), C.c_int()
         _check(lib().psvfwi_kernel_timing(self._h, k, C.byref(a), C.byref(b), C.byref(n)))
         return a.value, b.value, n.value
+
+    def last_step(self, kind):
+        """(tile, gave_up) of the last 'forward' or 'adjoint' run: tile 0 for the resident time loop,
+        else the set_tile value; gave_up: the plan keeps off the loop until set_tile(0)."""
+        tile, gave = C.c_int(), C.c_int()
+        _check(lib().psvfwi_last_step(self._h, {"forward": 0, "adjoint": 1}[kind], C.byref(tile), C.byref(gave)))
+        return tile.value, bool(gave.value)
 
 
 def parabola_step(L2, steps):

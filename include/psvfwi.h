@@ -290,6 +290,14 @@ psvfwi_status psvfwi_last_timing(const psvfwi_plan* plan, double* ms, long* laun
 psvfwi_status psvfwi_kernel_timing(const psvfwi_plan* plan, int kind, double* us_stress,
                                    double* us_velocity, int* samples);
 
+/* What the last forward (kind 0) or adjoint (kind 1) call ran on: *tile 0 for the resident time
+ * loop, else the psvfwi_set_tile value of the step.  *gave_up: 1 where the plan keeps to the
+ * other steps because a launch of the resident loop was refused or a wait in it ran out after
+ * about two seconds (kernels of another process that hold the GPU that long); that run was done
+ * again, and psvfwi_set_tile(plan, 0) lets the plan try the loop once more.  Either pointer may
+ * be NULL; PSVFWI_E_STATE before the first such call.  (No counterpart in the reference.) */
+psvfwi_status psvfwi_last_step(const psvfwi_plan* plan, int kind, int* tile, int* gave_up);
+
 /* ---- host-side setup (FP64): the inputs the kernels read ---- */
 
 /* hc[0..6] for FD order 2..12 and error class 0..4: holbergcoeff

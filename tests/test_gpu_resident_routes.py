@@ -1,0 +1,80 @@
+"""Which step a run takes: the resident time loop or the step kernels, and that every caller's
+route gives the split step's results bit for bit."""
+import numpy as np
+import pytest
+
+import psv_oracle as O
+import refcase as RC
+from cuda_fwi_amd import psvfwi as P
+from gpucase import plan_of, shots_of
+from test_gpu_resident import CASES, _problem, _same
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: f"{c[0]}x{c[1]}p{c[2]}o{c[3]}fs{c[4]}{c[5]}K{c[7]}")
+def test_exact_gradient_takes_the_resident_loop(case):
+    """The replay and the transposed steps of every shape are built and chosen: what the equality
+    with the split step is about."""
+    print(f"route of the exact gradient {case}", flush=True)
+    pb, shots, obs = _problem(case, 2, dict(dt=1))
+    plan = plan_of(pb, case[5], shots=shots)
+    plan.set_gradient_mode("discrete", max(8, case[6] // 2 - 3))
+    plan.forward(gradient=True)
+    plan.misfit(obs)
+    plan.adjoint(gradient=True)
+    assert plan.last_step("forward") == (0, False)
+    assert plan.last_step("adjoint") == (0, False)
+    plan.close()
+
+
+def test_last_step_names_the_step():
+    print("last step", flush=True)
+    pb = RC.small_problem(nx=60, nz=40, npml=8, nt=40, fdorder=4)
+    plan = plan_of(pb, "fp32", tz=-16)
+    with pytest.raises(P.PsvfwiError) as e:
+        plan.last_step("forward")
+    assert e.value.status == -5
+    for tz in (-16, 4, 0):
+        plan.set_tile(tz)
+        plan.forward()
+        assert plan.last_step("forward") == (tz, False)
+    with pytest.raises(P.PsvfwiError):
+        plan.last_step("adjoint")
+    plan.close()
+
+
+@pytest.mark.parametrize("prec", ["fp32", "fp64"])
+def test_rounds_of_several_shots(prec):
+    """More shots than one launch holds: rounds of several shots, the last one not full, records
+    of uneven length."""
+    print(f"rounds of shots {prec}", flush=True)
+    base = RC.small_problem(nx=200, nz=100, npml=40, nt=10, fdorder=4, fsurf=0, hetero=True)
+    shots, obs = [], []
+    rng = np.random.default_rng(8)
+    for i in range(19):
+        nt = 40 + 3 * (i * 7 % 19)
+        sig = O.create_wavelet(nt, base.dt, 1.0 + i, 25.0, 0.0)[None]
+        shots.append(dict(nt=nt, src=dict(x=[60 + 9 * i], z=[base.ppad + 4 + i], comp=[2]), src_signal=sig,
+                          rec=dict(x=[58 + 9 * i, 140, 150], z=[base.ppad + 3 + i] * 3, comp=[2, 1, 2])))
+        obs.append(rng.standard_normal((3, nt)) * 1e-3)
+    out = []
+    for tz in (8, None):
+        plan = plan_of(base, prec, tz=tz, shots=shots)
+        r = []
+        for mode in (("full", 0), ("checkpoint", 17), "discrete"):
+            plan.set_window(RC.full_window(base, dt=2))
+            if mode == "discrete":
+                plan.set_gradient_mode("discrete", 30)
+            else:
+                plan.set_store_mode(*mode)
+            plan.forward(gradient=True)
+            r += [plan.records(i) for i in range(19)] + [plan.misfit(obs)]
+            plan.adjoint(gradient=True)
+            r += list(plan.model_gradient(-1) if mode == "discrete" else plan.gradient(-1))
+            for kind in ("forward", "adjoint"):
+                assert plan.last_step(kind) == (tz or 0, False)
+        plan.close()
+        out.append(r)
+    assert all(np.abs(a).max() > 0 for a in out[0])
+    assert all(_same(a, b) for a, b in zip(*out))
