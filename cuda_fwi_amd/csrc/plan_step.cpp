@@ -62,9 +62,45 @@ psvfwi_status Plan<T>::autotune(int steps, int* best)
         *out = ms;
         return PSVFWI_OK;
     };
+    // the shot-to-workgroup order of a batch: shot-major, or bands of 1 or
+    // 4 tile rows with the shots of a band together; then the shots per launch
+    // group (split step only): the whole batch, or groups small enough for their
+    // wavefields to stay in the Infinity Cache between steps
+    auto tune_batch = [&](float* best_ms) -> psvfwi_status {
+        if (nslots_ < 2) return PSVFWI_OK;
+        int best_band = band_;
+        const int bands[3] = {0, 1, 4};
+        for (int b : bands) {
+            band_ = b;
+            float ms = 0;
+            PSV_TRY(time_steps(&ms));
+            if (b == 0 || ms < *best_ms) {
+                *best_ms = ms;
+                best_band = b;
+            }
+        }
+        band_ = best_band;
+        if (fused()) return PSVFWI_OK;
+        int best_lg = 0;
+        const int sizes[6] = {16, 12, 8, 6, 4, 2};
+        lg_ = 0;
+        PSV_TRY(time_steps(best_ms));
+        for (int k : sizes) {
+            if (k >= nslots_) continue;
+            lg_ = k;
+            float ms = 0;
+            PSV_TRY(time_steps(&ms));
+            if (ms < *best_ms) {
+                *best_ms = ms;
+                best_lg = k;
+            }
+        }
+        lg_ = best_lg;
+        return PSVFWI_OK;
+    };
     const int cand[kNumCand] = {4, 8, 16, 32, -8, -16, -32, -64};
-    float best_ms = 1e30f;
-    int best_tz = tz_;
+    float best_ms = 1e30f, split_ms = 1e30f;
+    int best_tz = tz_, split_tz = kDefaultTz;
     // the resident loop first, where it fits: over four times the steps, of which a launch's
     // reading and writing of the state is a small part, as in a run
     float res_ms = 1e30f;
@@ -108,49 +144,23 @@ psvfwi_status Plan<T>::autotune(int steps, int* best)
             best_ms = ms;
             best_tz = tz_;
         }
+        if (tz_ > 0 && ms < split_ms) {
+            split_ms = ms;
+            split_tz = tz_;
+        }
     }
     tz_ = best_tz;
-    // the shot-to-workgroup order of a batch: shot-major, or bands of 1 or
-    // 4 tile rows with the shots of a band together
-    if (nslots_ > 1) {
-        int best_band = band_;
-        const int bands[3] = {0, 1, 4};
-        for (int b : bands) {
-            band_ = b;
-            float ms = 0;
-            PSV_TRY(time_steps(&ms));
-            if (b == 0 || ms < best_ms) {
-                best_ms = ms;
-                best_band = b;
-            }
-        }
-        band_ = best_band;
-        // shots per launch group (split step only): the whole batch, or
-        // groups small enough for their wavefields to stay in the
-        // Infinity Cache between steps
-        if (!fused()) {
-            int best_lg = 0;
-            const int sizes[6] = {16, 12, 8, 6, 4, 2};
-            lg_ = 0;
-            PSV_TRY(time_steps(&best_ms));
-            for (int k : sizes) {
-                if (k >= nslots_) continue;
-                lg_ = k;
-                float ms = 0;
-                PSV_TRY(time_steps(&ms));
-                if (ms < best_ms) {
-                    best_ms = ms;
-                    best_lg = k;
-                }
-            }
-            lg_ = best_lg;
-        }
-    }
+    PSV_TRY(tune_batch(&best_ms));
     // the resident loop stays the plan's choice (as set_tile(0) makes it) where it was the
-    // fastest; the value returned is the split or fused step's either way
-    tile_auto_ = res_ms < best_ms;
-    if (tile_auto_) tz_ = kDefaultTz;
-    if (best) *best = tile_auto_ ? kDefaultTz : best_tz;
+    // fastest.  The runs that cannot take it (snapshots, the random-boundary adjoint, short
+    // segments) then have the fastest split step, not the default: a fused one would swap the
+    // loop's state (64 x 64 FP64, forward and adjoint: tiles of 4 rows 2.07 ms, of 8 rows 2.78)
+    if (res_ms < best_ms) {
+        tile_auto_ = true;
+        tz_ = split_tz;
+        if (best_tz != split_tz) PSV_TRY(tune_batch(&split_ms));
+    }
+    if (best) *best = best_tz;
     // the candidates ran in the plan's own state, store and gradient buffers
     drop_results();
     return PSVFWI_OK;

@@ -145,13 +145,15 @@ psvfwi_status psvfwi_set_tile(psvfwi_plan* plan, int tz);
 
 /* Autotuner: times `steps` forward steps of the current batch with the
  * resident time loop (over up to four times the steps) and with every
- * step kernel and tile height of psvfwi_set_tile, keeps the fastest and
- * returns its psvfwi_set_tile value in *best_tile (may be NULL; 8 where the
- * resident loop was the fastest, which psvfwi_set_tile(plan, 0) asks for and
- * psvfwi_set_tile(plan, 8) rules out); for a batch it
- * then chooses the shot order (psvfwi_set_shot_order) and, with the split
- * step, the launch group (psvfwi_set_launch_group) the same way.  In the
- * random-boundary store mode only the split kernels (tz > 0) are tried.
+ * step kernel and tile height of psvfwi_set_tile and keeps the fastest.
+ * *best_tile (may be NULL) is the psvfwi_set_tile value of the fastest step
+ * kernel.  Where the resident loop was faster still, the plan keeps to that
+ * (as after psvfwi_set_tile(plan, 0)), with the fastest split kernels for the
+ * runs that cannot take it; setting *best_tile then would rule the loop out.
+ * For a batch it then chooses the shot order (psvfwi_set_shot_order) and,
+ * with the split step, the launch group (psvfwi_set_launch_group) the same
+ * way.  In the random-boundary store mode no fused or z-marching kernel is
+ * tried (the adjoint needs the split ones, tz > 0).
  * Needs set_model / set_pml / set_shots first.  (No counterpart in the
  * reference, whose launch shape is fixed at 16 x 16,
  * CUDA_week2/forward_kernel_PSV_GPU.cu:543-545.) */
