@@ -308,10 +308,11 @@ psvfwi_status Plan<T>::resident_points(Tables& t)
     return PSVFWI_OK;
 }
 
-// the tiles of the resident loop, on the device
+// the tiles of the resident loop, on the device; the start of a run
 template <typename T>
 psvfwi_status Plan<T>::resident_prepare()
 {
+    *res_.aborted = 0;  // (a run that ended with another error may have left it set)
     if (!res_.uploaded) {
         PSV_HIP(res_.tiles.alloc(res_.part.h.size()));
         PSV_HIP(hipMemcpy(res_.tiles.p, res_.part.h.data(), res_.part.h.size() * sizeof(psv::ResTile), hipMemcpyHostToDevice));
@@ -348,6 +349,7 @@ psvfwi_status Plan<T>::launch_resident(State<T>& st, Tables& tab, bool fwd_sig, 
     a.xpitch = res_.xpitch;
     a.zpitch = res_.zpitch;
     a.aborted = res_.aborted;
+    a.polls = res_.polls;
     a.kdiv = res_.kdiv;
     T** const in[psv::kStateArrays] = {&a.p.vx, &a.p.vz, &a.p.sxx, &a.p.szx, &a.p.szz, &a.p.mvxx, &a.p.mvzx,
                                        &a.p.msxxx, &a.p.mszxx, &a.p.mvzz, &a.p.mvxz, &a.p.mszzz, &a.p.mszxz};
@@ -382,7 +384,12 @@ psvfwi_status Plan<T>::launch_resident(State<T>& st, Tables& tab, bool fwd_sig, 
             a.pts.off = tab.res_off.p + ((size_t)w0_ * res_.part.h.size() + (size_t)t0) * res_.waves;
             a.tag = res_.tag;
             res_.tag += span;
-            e = psv::launch_resident<T>(a, g_.fdorder, mode, res_.shape, stream_);
+            if (res_.refuse > 0) {
+                res_.refuse--;
+                e = hipErrorCooperativeLaunchTooLarge;
+            } else {
+                e = psv::launch_resident<T>(a, g_.fdorder, mode, res_.shape, stream_);
+            }
         }
         if (nstrip > 1)
             for (int k = 0; k < psv::kStateArrays; k++) std::swap(*in[k], a.out[k]);
@@ -430,7 +437,19 @@ bool Plan<T>::resident_failed()
     return true;
 }
 
+// For tests: how long a wait lasts, the tag of the next launch (only up: the exchange buffer holds
+// the ones before it), and how many launches are refused.
+template <typename T>
+psvfwi_status Plan<T>::test_resident(unsigned polls, unsigned tag, int refuse)
+{
+    res_.polls = polls ? polls : psv::kResPolls;
+    res_.tag = std::max(res_.tag, tag);
+    res_.refuse = refuse;
+    return PSVFWI_OK;
+}
+
 #define PSV_INSTANTIATE(T) \
+    template psvfwi_status Plan<T>::test_resident(unsigned, unsigned, int); \
     template Plan<T>::Partition Plan<T>::resident_tiles(const psv::ResShape&, bool, int, int) const; \
     template bool Plan<T>::resident_ready(); \
     template size_t Plan<T>::resident_terms() const; \

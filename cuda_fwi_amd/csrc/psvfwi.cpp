@@ -335,6 +335,12 @@ psvfwi_status psvfwi_last_step(const psvfwi_plan* plan, int kind, int* tile, int
     return plan->last_step(kind, tile, gave_up);
 }
 
+psvfwi_status psvfwi_test_resident(psvfwi_plan* plan, unsigned polls, unsigned tag, int refuse)
+{
+    PSV_PLAN(plan);
+    return plan->test_resident(polls, tag, refuse);
+}
+
 psvfwi_status psvfwi_parabola_step(const double* L2, const double* step, double* opt)
 {
     if (!L2 || !step || !opt) return fail(PSVFWI_E_ARG, "parabola_step: null argument");

@@ -39,7 +39,7 @@ EXPORTS = ("psvfwi_last_error", "psvfwi_plan_create", "psvfwi_plan_destroy", "ps
            "psvfwi_set_gradient_mode", "psvfwi_get_coefficient_gradient", "psvfwi_get_model_gradient",
            "psvfwi_chain_gradient", "psvfwi_random_boundary", "psvfwi_set_shot_order",
            "psvfwi_get_shot_order", "psvfwi_set_launch_group", "psvfwi_get_launch_group",
-           "psvfwi_misfit_noalloc", "psvfwi_last_step")
+           "psvfwi_misfit_noalloc", "psvfwi_last_step", "psvfwi_test_resident")
 
 
 class PsvfwiError(RuntimeError):
@@ -348,6 +348,10 @@ class Plan:
         tile, gave = C.c_int(), C.c_int()
         _check(lib().psvfwi_last_step(self._h, {"forward": 0, "adjoint": 1}[kind], C.byref(tile), C.byref(gave)))
         return tile.value, bool(gave.value)
+
+    def test_resident(self, polls=0, tag=0, refuse=0):
+        """For tests: tries of a wait of the resident loop, its next exchange tag, launches refused."""
+        _check(lib().psvfwi_test_resident(self._h, C.c_uint(polls), C.c_uint(tag), int(refuse)))
 
 
 def parabola_step(L2, steps):
