@@ -174,8 +174,11 @@ template <typename T>
 class Plan final : public psvfwi_plan {
 public:
     static constexpr int kDefaultTz = 8;
-    // fewest steps a resident launch is worth: it loads the whole state and writes it back
+    // fewest steps of a segment that a resident launch is worth: it loads the whole state and
+    // writes it back
     static constexpr int kResidentMin = 8;
+    // ... and from where on the length of a run or segment does not matter
+    static constexpr int kResidentLong = 64;
 
     // ---------------------------------------------------------- plan_setup.cpp
     explicit Plan(const psvfwi_grid_desc& g);
@@ -262,6 +265,8 @@ private:
         bool want = false;      // chosen for a plan with the exact gradient ...
         bool discrete = false;  // ... and its shape has the replay and the reverse steps
         bool uploaded = false;
+        double us = 0, cells = 0;  // what a step takes, and M cells of a launch's tiles
+        int rounds = 0;            // launches a step
         int kdiv = 0;           // some CPML K differs from 1
         Partition part;
         DBuf<T> other[psv::kStateArrays];  // more strips: a slot's state after their steps
@@ -314,6 +319,7 @@ private:
     size_t resident_terms() const;
     bool chain_upload() const;
     bool resident_ready();
+    bool resident_for(int steps, bool forward, bool adjoint);
     psvfwi_status resident_points(Tables& t);
     psvfwi_status resident_prepare();
     psvfwi_status launch_resident(State<T>& st, Tables& tab, bool fwd_sig, int mode, int kind, int it0, int it1,

@@ -66,7 +66,9 @@ psvfwi_status Plan<T>::adjoint(int flags)
     const bool ckpt = grad && store_mode_ == PSVFWI_STORE_CHECKPOINT;
     if (grad && !ckpt && !store_loaded_) return fail(PSVFWI_E_STATE, "adjoint: forward store missing");
 
-    const bool resident = !(ckpt && ck_used_k_ < kResidentMin) && resident_ready();
+    // (checkpoints: the replay of a segment too)
+    const bool resident = !(ckpt && ck_used_k_ < kResidentMin) &&
+                          resident_for(ckpt ? std::min(ck_used_k_, ntmax_) : ntmax_, ckpt, true);
     if (resident) PSV_TRY(resident_prepare());
     const int gsize = resident ? res_.conc : group_size();
     PSV_TRY(alloc_state(main_));

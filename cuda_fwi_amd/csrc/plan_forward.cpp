@@ -37,7 +37,8 @@ psvfwi_status Plan<T>::forward(int flags)
     if (ckpt) PSV_TRY(alloc_checkpoints(every ? 0 : kint));
     const bool snap = snap_interval_ > 0;
     // short checkpoint intervals and snapshots need the state in memory after every few steps
-    const bool resident = !snap && !every && !(ckpt && kint < kResidentMin) && resident_ready();
+    const bool resident = !snap && !every && !(ckpt && kint < kResidentMin) &&
+                          resident_for(ckpt ? std::min(kint, ntmax_) : ntmax_, true, false);
     if (resident) PSV_TRY(resident_prepare());
     const int gsize = resident ? res_.conc : group_size();
     if (snap) PSV_HIP(snaps_.alloc((size_t)((ntmax_ - 1) / snap_interval_ + 1) * nslots_ * fst_));

@@ -139,6 +139,55 @@ static double strip_move_us(double cells, int esize, int steps)
     return (20.0 + cells * 15 * esize / 4e6) / steps;
 }
 
+// The forward and the adjoint step apart, for runs of few steps.  Split, us a step of `cells` M cells:
+// FP32 forward 11.1 on 0.06, 16.3 on 0.63, 38 on 2.2, 92 on 6.6, adjoint 11.7, 17.8, 45, 122; FP64
+// forward 13.8 on 0.008, 31 on 0.81, 65 on 2.2, adjoint 14.0, 36, 79; compensated FP32 18 on 0.06,
+// 34 on 0.45.
+static double split_us(double cells, int esize, bool dwords, bool forward)
+{
+    if (dwords) return 16.5 + 38.0 * cells;
+    return esize == 4 ? std::max(11.0, 9.0 + (forward ? 12.9 : 17.0) * cells) : 12.0 + (forward ? 23.5 : 31.0) * cells;
+}
+
+// A launch of the resident loop besides its steps, us, where its tiles have `cells` M cells: it
+// starts, loads the state and the model and writes the state back.  Measured FP32 forward 21 on 0.06,
+// 28 on 0.63, 40 on 1.08, and a strip's 43 on 1.4, 50 on 1.6, adjoint 21, 37, 54, 72, 80; FP64 forward
+// 27 on 0.26, 36 on 0.41, a strip's 51 on 0.85, adjoint 32, 46, 66.
+static double launch_us(double cells, int esize, bool forward)
+{
+    return 20.0 + cells * esize / 4 * (forward ? (esize == 4 ? 17.0 : 16.0) : (esize == 4 ? 36.0 : 25.0));
+}
+
+// Whether the resident loop pays in a run of records or segments of `steps` steps that are run
+// forward, backward or (the replay of a segment) both.  A strip's launches are half a segment long at
+// most.  The line lies where the two sums meet: 8 steps of 3600 x 1200 in FP32, forward, 0.61 ms
+// resident and 0.55 split (12 steps 0.71, 0.81); checkpoints 8 apart there, replay and adjoint of 96
+// steps, 19.4 and 16.2 ms (12 apart 15.1, 16.1); 600 x 300 in FP64, adjoint, 2 steps 0.059 and 0.054
+// (3 steps 0.060, 0.074).
+template <typename T>
+bool Plan<T>::resident_for(int steps, bool forward, bool adjoint)
+{
+    constexpr bool dwords = std::is_same<T, psv::dfloat>::value;
+    constexpr int esize = (int)sizeof(T);
+    const double all = 1e-6 * nslots_ * g_.nzt * g_.nxt;
+    double split = 0, least = 0;
+    for (bool f : {true, false})
+        if (f ? forward : adjoint) {
+            split += split_us(all, esize, dwords, f);
+            least += 2.9 + launch_us(all, esize, f) / steps;
+        }
+    // (no search for a shape where none could pay)
+    if (steps < kResidentLong && least >= split) return false;
+    if (!resident_ready()) return false;
+    if (steps >= kResidentLong) return true;
+    const int most = res_.part.strips.size() > 2 ? std::min(res_.part.steps, (steps + 1) / 2) : steps;
+    double cost = 0;
+    for (bool f : {true, false})
+        if (f ? forward : adjoint)
+            cost += res_.rounds * (res_.us * (f || esize == 8 ? 1.0 : 1.15) + launch_us(res_.cells, esize, f) / most);
+    return cost < split;
+}
+
 // Whether the plan's runs can take the resident loop, and its shape for the current batch.
 // Not for a caller who chose a tile height; not for CPML profiles that couple the strips
 // (the reference's arrays give the innermost cells of the two strips of an axis one memory
@@ -184,6 +233,8 @@ bool Plan<T>::resident_ready()
             const double cost = rounds * (shapes[i].us + move);
             if (cost < best) {
                 best = cost;
+                res_.us = shapes[i].us;
+                res_.rounds = rounds;
                 res_.shape = i;
                 res_.conc = conc;
                 res_.cap = cap;
@@ -205,6 +256,9 @@ bool Plan<T>::resident_ready()
             break;
         }
     }
+    res_.cells = 0;
+    for (const psv::ResTile& t : res_.part.h) res_.cells += (double)(t.z1 - t.z0) * (t.x1 - t.x0);
+    res_.cells *= 1e-6 * (res_.part.strips.size() > 2 ? 1.0 / (res_.part.strips.size() - 1) : res_.conc);
     // the exchange buffer, the flag, and for strips the other set of a slot's state
     {
         res_.xpitch = (int)round_up((size_t)g_.nxt, 8);
@@ -452,6 +506,7 @@ psvfwi_status Plan<T>::test_resident(unsigned polls, unsigned tag, int refuse)
     template psvfwi_status Plan<T>::test_resident(unsigned, unsigned, int); \
     template Plan<T>::Partition Plan<T>::resident_tiles(const psv::ResShape&, bool, int, int) const; \
     template bool Plan<T>::resident_ready(); \
+    template bool Plan<T>::resident_for(int, bool, bool); \
     template size_t Plan<T>::resident_terms() const; \
     template psvfwi_status Plan<T>::resident_points(Tables&); \
     template psvfwi_status Plan<T>::resident_prepare(); \

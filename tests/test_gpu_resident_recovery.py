@@ -11,15 +11,15 @@ from test_gpu_resident import _problem, _same
 pytestmark = pytest.mark.gpu
 
 # nx, nz, npml, order, fsurf, precision, nt, K: several tiles; strips
-GRIDS = [(101, 77, 8, 4, 1, "fp32", 60, 1.0), (160, 120, 10, 2, 0, "fp64", 45, 1.0), (1900, 700, 20, 4, 0, "fp32", 24, 1.0)]
+GRIDS = [(101, 77, 8, 4, 1, "fp32", 60, 1.0), (160, 120, 10, 2, 0, "fp64", 45, 1.0), (1900, 700, 20, 4, 0, "fp32", 70, 1.0)]
 FORCE = {"wait": dict(polls=1), "refused": dict(refuse=1)}
 
 
 def _setup(plan, mode):
     if mode == "discrete":
-        plan.set_gradient_mode("discrete", 11)
+        plan.set_gradient_mode("discrete", 31)
     else:
-        plan.set_store_mode(mode, 9)
+        plan.set_store_mode(mode, 29)
 
 
 def _forward(plan):

@@ -117,3 +117,30 @@ def test_autotuned_tile_serves_the_runs_the_loop_cannot():
     ref.misfit(obs)
     ref.adjoint()
     assert all(_same(a, b) for a, b in zip(g, ref.gradient()))
+
+
+@pytest.mark.parametrize("grid,segments,short,long", [((84, 84, 0, 4, 0, "fp64"), False, 2, 16),
+                                                      ((1900, 700, 20, 4, 0, "fp32"), False, 4, 16),
+                                                      ((2400, 800, 20, 4, 1, "fp64"), True, 8, 32)],
+                         ids=lambda g: "x".join(map(str, g)) if isinstance(g, tuple) else str(g))
+def test_short_runs_stay_on_the_split_step(grid, segments, short, long):
+    """A resident launch loads and writes the whole state: records of a step or two, and on grids in
+    strips of a few steps, and segments of 8 there, are faster on the split step.  Either way the same
+    results."""
+    print(f"short runs {grid}", flush=True)
+    pb, shots, obs = _problem(grid + (48, 1.0), 2, dict(dt=2))
+    for k in (short, long):
+        nt = pb.nt if segments else k
+        one = dict(shots[0], nt=nt, src_signal=shots[0]["src_signal"][:, :nt])
+        out = []
+        for tz in (8, None):
+            plan = plan_of(pb, grid[5], tz=tz, shots=[one])
+            plan.set_store_mode("checkpoint" if segments else "full", k)
+            plan.forward(gradient=True)
+            r = [plan.records(), plan.misfit([obs[0][:, :nt]])]
+            plan.adjoint()
+            out.append(r + list(plan.gradient()))
+            want = 8 if tz or k == short else 0
+            assert [plan.last_step(q)[0] for q in ("forward", "adjoint")] == [want, want], k
+            plan.close()
+        assert all(_same(a, b) for a, b in zip(*out))
