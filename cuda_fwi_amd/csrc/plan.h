@@ -37,6 +37,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <initializer_list>
 #include <numeric>
 #include <string>
 #include <vector>
@@ -321,7 +322,7 @@ private:
     bool resident_ready();
     bool resident_for(int steps, bool forward, bool adjoint);
     psvfwi_status resident_points(Tables& t);
-    psvfwi_status resident_prepare();
+    psvfwi_status resident_prepare(std::initializer_list<Tables*> tabs);
     psvfwi_status launch_resident(State<T>& st, Tables& tab, bool fwd_sig, int mode, int kind, int it0, int it1,
                                   int flags, int tf0, bool one_plane = false);
     bool resident_failed();

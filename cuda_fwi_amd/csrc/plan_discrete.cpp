@@ -33,7 +33,7 @@ psvfwi_status Plan<T>::adjoint_discrete()
     const bool every = kk == 1;
     bool resident = kk >= kResidentMin && resident_ready() && res_.discrete;
     if (resident) {
-        PSV_TRY(resident_prepare());
+        PSV_TRY(resident_prepare({&adj_tab_, &fwd_tab_noreceivers_}));
         PSV_TRY(alloc_state(replay_));
         // (the terms of a segment may need more memory than its states: then the split step)
         if (seg_.reserve((size_t)std::min(kk, ntmax_) * res_.conc * resident_terms()) != hipSuccess) {

@@ -39,7 +39,7 @@ psvfwi_status Plan<T>::forward(int flags)
     // short checkpoint intervals and snapshots need the state in memory after every few steps
     const bool resident = !snap && !every && !(ckpt && kint < kResidentMin) &&
                           resident_for(ckpt ? std::min(kint, ntmax_) : ntmax_, true, false);
-    if (resident) PSV_TRY(resident_prepare());
+    if (resident) PSV_TRY(resident_prepare({&fwd_tab_}));
     const int gsize = resident ? res_.conc : group_size();
     if (snap) PSV_HIP(snaps_.alloc((size_t)((ntmax_ - 1) / snap_interval_ + 1) * nslots_ * fst_));
     snaps_taken_ = snap;

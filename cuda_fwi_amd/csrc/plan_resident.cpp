@@ -362,9 +362,9 @@ psvfwi_status Plan<T>::resident_points(Tables& t)
     return PSVFWI_OK;
 }
 
-// the tiles of the resident loop, on the device; the start of a run
+// the tiles of the resident loop and the point tables of a run, on the device before its timed part
 template <typename T>
-psvfwi_status Plan<T>::resident_prepare()
+psvfwi_status Plan<T>::resident_prepare(std::initializer_list<Tables*> tabs)
 {
     *res_.aborted = 0;  // (a run that ended with another error may have left it set)
     if (!res_.uploaded) {
@@ -372,6 +372,7 @@ psvfwi_status Plan<T>::resident_prepare()
         PSV_HIP(hipMemcpy(res_.tiles.p, res_.part.h.data(), res_.part.h.size() * sizeof(psv::ResTile), hipMemcpyHostToDevice));
         res_.uploaded = true;
     }
+    for (Tables* t : tabs) PSV_TRY(resident_points(*t));
     return PSVFWI_OK;
 }
 
@@ -381,7 +382,6 @@ template <typename T>
 psvfwi_status Plan<T>::launch_resident(State<T>& st, Tables& tab, bool fwd_sig, int mode, int kind, int it0, int it1,
                                        int flags, int tf0, bool one_plane)
 {
-    PSV_TRY(resident_points(tab));
     const int steps = it1 - it0;
     psv::ResidentParams<T> a{};
     if (mode >= psv::kReplay) {
@@ -509,7 +509,7 @@ psvfwi_status Plan<T>::test_resident(unsigned polls, unsigned tag, int refuse)
     template bool Plan<T>::resident_for(int, bool, bool); \
     template size_t Plan<T>::resident_terms() const; \
     template psvfwi_status Plan<T>::resident_points(Tables&); \
-    template psvfwi_status Plan<T>::resident_prepare(); \
+    template psvfwi_status Plan<T>::resident_prepare(std::initializer_list<Tables*>); \
     template psvfwi_status Plan<T>::launch_resident(State<T>&, Tables&, bool, int, int, int, int, int, int, bool); \
     template bool Plan<T>::resident_failed();
 PSV_FOR_EACH_PRECISION(PSV_INSTANTIATE)

@@ -107,7 +107,7 @@ psvfwi_status Plan<T>::autotune(int steps, int* best)
     tile_auto_ = true;
     if (resident_ready()) {
         tz_ = kDefaultTz;
-        PSV_TRY(resident_prepare());
+        PSV_TRY(resident_prepare({&adj_tab_, &fwd_tab_noreceivers_}));
         AllSlotsAfter restore{this};
         for (int rep = 0; rep < 2; rep++) {
             PSV_TRY(zero_state(main_));
