@@ -135,6 +135,14 @@ def step_kernel_name(plan_tile, resident):
             "fused tile" if plan_tile > -32 else "z-marching segments")
 
 
+def step_config(plan):
+    """The step kernel, tile and launch group of a plan's last adjoint run; the resident time loop has
+    neither tile nor group."""
+    tile = plan.last_step("adjoint")[0]
+    return {"step_kernel": step_kernel_name(tile, tile == 0), "tile": [64, abs(tile)] if tile else None,
+            "launch_group": (plan.launch_group() or "whole batch") if tile else None}
+
+
 def cpu_baseline(w, window, nt_sample, threaded=False):
     """The oracle (FP64 CPU restatement of the reference path) on the same
     grid, model and geometry, for nt_sample steps: single-threaded (the
@@ -281,7 +289,7 @@ def run_c2(args):
                                       "(no CPML: the outer 40 cells hold a random layer)"}.get(
                                           args.store, f"checkpoint every {args.interval}"),
                    "fwi_time_decimation": fwi_dt,
-                   "tile": [64, abs(plan.tile)],
+                   "tile": None if resident else [64, abs(plan.tile)],
                    "step_kernel": step_kernel_name(plan.tile, resident),
                    "tile_choice": "autotuned" if args.tile == 0 else "fixed",
                    "graph_steps": args.graph_steps},
@@ -356,7 +364,7 @@ def run_c2_discrete(args):
                 "the unperturbed layers (synthetic)",
         "config": {"workload": f"1000x500 dx5 order-4 npml40, nt {w.nt}, dt 0.4 ms, 1 shot, 400 receivers, "
                                "fwd+adj+grad with the discrete (exact) gradient on the whole grid",
-                   "checkpoint_interval": args.interval, "tile": [64, abs(plan.tile)]},
+                   "checkpoint_interval": args.interval, **step_config(plan)},
         "forward_ms_per_step": round(tf / args.steps, 2),
         "adjoint_ms_per_step": round(ta / args.steps, 2),
     }
@@ -458,8 +466,7 @@ def run_c5(args):
                                + (", preconditioner sqrt(Ws Wr)" if args.c5_precond == "source_receiver" else "")
                                + (f", cosine taper over {args.c5_taper} rows" if args.c5_taper > 0 else "")
                                + (f", depth gain power {args.c5_depth_power:g}" if args.c5_depth_power > 0 else ""),
-                   "scale_of_2400x800_128_shots": sc, "tile": plan.tile,
-                   "launch_group": plan.launch_group() or "whole batch"},
+                   "scale_of_2400x800_128_shots": sc, **step_config(plan)},
         "fwi": {"misfit": prev["misfit"], "vp_rel_error_start": err0, "vp_rel_error": prev["model_error"],
                 "vp_rel_error_lowpass": {f"sigma {sig:g} cells": {"start": a, "end": inv.model_error(truth, sig)}
                                          for sig, a in zip(sigmas, low0)},
@@ -697,9 +704,11 @@ def run_c4(args):
                                       f"{args.store_budget_gb} GB of store" if args.store == "full" else
                                       f"checkpoint every {args.interval} steps, segments recomputed "
                                       "(recomputation not counted)"),
-                   "tile": tile, "step_kernel": step_kernel_name(tile, resident),
-                   "shot_order": "shot-major" if band == 0 else f"bands of {band} tile rows",
-                   "launch_group": lgroup or "whole group", "graph_steps": args.graph_steps},
+                   "step_kernel": step_kernel_name(tile, resident),
+                   # (of the step kernels: the resident loop runs as many shots as fit, without these)
+                   "tile": None if resident else tile,
+                   "shot_order": None if resident else ("shot-major" if band == 0 else f"bands of {band} tile rows"),
+                   "launch_group": None if resident else lgroup or "whole group", "graph_steps": args.graph_steps},
         "roofline": {"bound": "rim exchange and instructions" if resident else "hbm",
                      "kernel": (RESIDENT_NAMES if resident else KERNEL_NAMES)[kname], "achieved": round(achieved, 1),
                      "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
@@ -834,7 +843,7 @@ def run_c3mem(args):
         "data": "synthetic: 8 flat layers", "config": {
             "workload": f"2000x1000 dx5 order-4, nt {w.nt}, 1 shot, fwd+adj+grad, " + (
                 "random-boundary reconstruction (no CPML: a 40-cell random layer)" if mode == "random_boundary"
-                else f"npml40, checkpoint every {args.interval} steps") + f", fwi_dt {fwi_dt}", "tile": plan.tile},
+                else f"npml40, checkpoint every {args.interval} steps") + f", fwi_dt {fwi_dt}", **step_config(plan)},
         "memory": {"device_used_before_GB": round((total - free0) / 1e9, 2),
                    "device_used_peak_GB": round(max(used) / 1e9, 2),
                    "device_total_GB": round(total / 1e9, 1),

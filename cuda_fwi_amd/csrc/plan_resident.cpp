@@ -41,8 +41,8 @@ std::vector<psv::ResTile> tile_column(int nzt, int zlo, int zhi, bool xin, int o
 
 }  // namespace
 
-// The tiles of the grid for a shape, in strips of at most `cap` (none: they do not fit).  Interior tiles: every stress cell they compute (2 cells around the owned ones)
-// is updated, outside the CPML strips and below the free-surface row; for the transposed steps also
+// The tiles of the grid for a shape, in strips of at most `cap` (none: they do not fit).
+// Interior tiles: every stress cell they compute (2 cells around the owned ones) is updated, outside the CPML strips and below the free-surface row; for the transposed steps also
 // every velocity weight they form (kResHalo cells around) is one of an updated cell outside the
 // strips, and none of their stress cells is mirrored.
 template <typename T>

@@ -138,10 +138,11 @@ psvfwi_status psvfwi_set_shots(psvfwi_plan* plan, int nshots, const psvfwi_shot_
  * the point sources and receivers; 0 = default: the resident time loop (many
  * steps in one launch, the wavefields in registers) where the precision, the
  * CPML profiles, the grid and the batch allow it and it is expected to be
- * faster, else two launches on tiles of 8 rows.  Random-boundary and
- * snapshot runs, checkpoints less than 8 steps apart, and runs or segments too
- * short to be worth loading the state (one or two steps; on grids of millions of
- * cells up to about 12) take the two launches.  Every choice gives the same results bit for bit. */
+ * faster, else two launches on tiles of 8 rows.  Random-boundary adjoints
+ * (the forward may be resident), snapshot runs, checkpoints less than 8 steps
+ * apart, and runs or segments too short to be worth loading the state (one or
+ * two steps; on grids of millions of cells up to about 12) take the two
+ * launches.  Every choice gives the same results bit for bit. */
 psvfwi_status psvfwi_set_tile(psvfwi_plan* plan, int tz);
 
 /* Autotuner: times `steps` forward steps of the current batch with the
@@ -173,8 +174,8 @@ psvfwi_status psvfwi_get_shot_order(const psvfwi_plan* plan, int* band);
  * before the next (slots are the shots sorted by decreasing nt), so that a group's
  * wavefields stay in the GPU's 256 MB Infinity Cache from one step to the next; 0 (default)
  * steps the whole batch together.  The fused step (tile < 0) always runs the batch as one
- * group, the resident time loop as many shots as fit in the registers.  psvfwi_autotune chooses among 0, 16, 12, 8, 6, 4 and 2 for batches.  Results do not
- * depend on it. */
+ * group, the resident time loop as many shots as fit in the registers.  psvfwi_autotune
+ * chooses among 0, 16, 12, 8, 6, 4 and 2 for batches.  Results do not depend on it. */
 psvfwi_status psvfwi_set_launch_group(psvfwi_plan* plan, int shots);
 psvfwi_status psvfwi_get_launch_group(const psvfwi_plan* plan, int* shots);
 
