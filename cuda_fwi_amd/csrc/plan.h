@@ -88,7 +88,7 @@ struct psvfwi_plan {
     virtual psvfwi_status timing(double*, long*) const = 0;
     virtual psvfwi_status kernel_timing(int, double*, double*, int*) const = 0;
     virtual psvfwi_status last_step(int, int*, int*) const = 0;
-    virtual psvfwi_status test_resident(unsigned, unsigned, int) = 0;
+    virtual psvfwi_status test_resident(int, unsigned, int) = 0;
 };
 
 namespace psvplan {
@@ -276,8 +276,8 @@ private:
         size_t exch_slot = 0;
         int xpitch = 0, zpitch = 0;
         unsigned tag = 1;
-        unsigned polls = psv::kResPolls;
-        int refuse = 0;          // launches still to be refused (test_resident)
+        int mute = 0;            // test_resident: a tile that is silent ...
+        int refuse = 0;          // ... launches still to be refused
         int* aborted = nullptr;  // pinned host memory the kernel writes when a wait runs out
     };
 
@@ -326,7 +326,7 @@ private:
     psvfwi_status launch_resident(State<T>& st, Tables& tab, bool fwd_sig, int mode, int kind, int it0, int it1,
                                   int flags, int tf0, bool one_plane = false);
     bool resident_failed();
-    psvfwi_status test_resident(unsigned polls, unsigned tag, int refuse) override;
+    psvfwi_status test_resident(int mute, unsigned tag, int refuse) override;
 
     // -------------------------------------------------------- plan_adjoint.cpp
     psvfwi_status adjoint_step(int it, int flags, int tf0);

@@ -366,11 +366,16 @@ psvfwi_status Plan<T>::resident_points(Tables& t)
 template <typename T>
 psvfwi_status Plan<T>::resident_prepare(std::initializer_list<Tables*> tabs)
 {
-    *res_.aborted = 0;  // (a run that ended with another error may have left it set)
-    if (!res_.uploaded) {
-        PSV_HIP(res_.tiles.alloc(res_.part.h.size()));
-        PSV_HIP(hipMemcpy(res_.tiles.p, res_.part.h.data(), res_.part.h.size() * sizeof(psv::ResTile), hipMemcpyHostToDevice));
-        res_.uploaded = true;
+    // (a run that ended with another error may have left it set; set before a run, waits are over
+    // after their first look at it)
+    *res_.aborted = res_.mute == 1;
+    if (!res_.uploaded || res_.mute) {
+        std::vector<psv::ResTile> h = res_.part.h;
+        // a tile at the edge of a strip has no neighbour there
+        if (res_.mute) h[0].xe = h[0].x1;
+        PSV_HIP(res_.tiles.alloc(h.size()));
+        PSV_HIP(hipMemcpy(res_.tiles.p, h.data(), h.size() * sizeof(psv::ResTile), hipMemcpyHostToDevice));
+        res_.uploaded = res_.mute == 0;
     }
     for (Tables* t : tabs) PSV_TRY(resident_points(*t));
     return PSVFWI_OK;
@@ -403,7 +408,6 @@ psvfwi_status Plan<T>::launch_resident(State<T>& st, Tables& tab, bool fwd_sig, 
     a.xpitch = res_.xpitch;
     a.zpitch = res_.zpitch;
     a.aborted = res_.aborted;
-    a.polls = res_.polls;
     a.kdiv = res_.kdiv;
     T** const in[psv::kStateArrays] = {&a.p.vx, &a.p.vz, &a.p.sxx, &a.p.szx, &a.p.szz, &a.p.mvxx, &a.p.mvzx,
                                        &a.p.msxxx, &a.p.mszxx, &a.p.mvzz, &a.p.mvxz, &a.p.mszzz, &a.p.mszxz};
@@ -491,19 +495,20 @@ bool Plan<T>::resident_failed()
     return true;
 }
 
-// For tests: how long a wait lasts, the tag of the next launch (only up: the exchange buffer holds
-// the ones before it), and how many launches are refused.
+// For tests: the first tile sends nothing to its right, so that the tiles there wait in vain (mute 1:
+// until their first look at `aborted`, 2: until they give up), the tag of the next launch (only up:
+// the exchange buffer holds the ones before it), and how many launches are refused.
 template <typename T>
-psvfwi_status Plan<T>::test_resident(unsigned polls, unsigned tag, int refuse)
+psvfwi_status Plan<T>::test_resident(int mute, unsigned tag, int refuse)
 {
-    res_.polls = polls ? polls : psv::kResPolls;
+    res_.mute = mute;
     res_.tag = std::max(res_.tag, tag);
     res_.refuse = refuse;
     return PSVFWI_OK;
 }
 
 #define PSV_INSTANTIATE(T) \
-    template psvfwi_status Plan<T>::test_resident(unsigned, unsigned, int); \
+    template psvfwi_status Plan<T>::test_resident(int, unsigned, int); \
     template Plan<T>::Partition Plan<T>::resident_tiles(const psv::ResShape&, bool, int, int) const; \
     template bool Plan<T>::resident_ready(); \
     template bool Plan<T>::resident_for(int, bool, bool); \

@@ -47,8 +47,6 @@ struct ResPoints {
     const int* id;    // [layer][64]
 };
 
-constexpr unsigned kResPolls = 1u << 21;  // tries of a wait: about two seconds
-
 // What a launch runs: the forward and adjoint steps (kForward, kAdjoint), and for the exact
 // gradient a forward segment that writes its derivative terms and the transposed steps that
 // read them back.
@@ -69,7 +67,6 @@ struct ResidentParams {
     int xpitch, zpitch;
     unsigned tag;            // tag of the launch's first step
     int* aborted;            // host memory: set when a wait ran out
-    unsigned polls;          // tries of a wait
     int kdiv;                // some CPML K differs from 1
     T* out[kStateArrays];    // the state after the steps: p's own arrays, or another set where
                              // strips still have to read the state before them

@@ -335,10 +335,10 @@ psvfwi_status psvfwi_last_step(const psvfwi_plan* plan, int kind, int* tile, int
     return plan->last_step(kind, tile, gave_up);
 }
 
-psvfwi_status psvfwi_test_resident(psvfwi_plan* plan, unsigned polls, unsigned tag, int refuse)
+psvfwi_status psvfwi_test_resident(psvfwi_plan* plan, int mute, unsigned tag, int refuse)
 {
     PSV_PLAN(plan);
-    return plan->test_resident(polls, tag, refuse);
+    return plan->test_resident(mute, tag, refuse);
 }
 
 psvfwi_status psvfwi_parabola_step(const double* L2, const double* step, double* opt)

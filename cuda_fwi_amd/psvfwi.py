@@ -349,9 +349,10 @@ class Plan:
         _check(lib().psvfwi_last_step(self._h, {"forward": 0, "adjoint": 1}[kind], C.byref(tile), C.byref(gave)))
         return tile.value, bool(gave.value)
 
-    def test_resident(self, polls=0, tag=0, refuse=0):
-        """For tests: tries of a wait of the resident loop, its next exchange tag, launches refused."""
-        _check(lib().psvfwi_test_resident(self._h, C.c_uint(polls), C.c_uint(tag), int(refuse)))
+    def test_resident(self, mute=0, tag=0, refuse=0):
+        """For tests of the resident loop: a tile that sends nothing to the right (waits run out, with 1
+        early), the next exchange tag, launches refused."""
+        _check(lib().psvfwi_test_resident(self._h, int(mute), C.c_uint(tag), int(refuse)))
 
 
 def parabola_step(L2, steps):

@@ -302,10 +302,11 @@ psvfwi_status psvfwi_kernel_timing(const psvfwi_plan* plan, int kind, double* us
  * be NULL; PSVFWI_E_STATE before the first such call.  (No counterpart in the reference.) */
 psvfwi_status psvfwi_last_step(const psvfwi_plan* plan, int kind, int* tile, int* gave_up);
 
-/* For tests of the resident loop's recovery, without a fault on the GPU: a wait gives up after
- * `polls` tries (0: the usual number), the exchange tags go on from `tag` where that is higher
- * (after a first run), and the next `refuse` launches are refused on the host. */
-psvfwi_status psvfwi_test_resident(psvfwi_plan* plan, unsigned polls, unsigned tag, int refuse);
+/* For tests of the resident loop's recovery, without a fault on the GPU: with mute 1 or 2 the first
+ * tile sends nothing to its neighbour on the right, so that waits run out (grids of more than 64
+ * columns), with 1 about a millisecond after the start; the exchange tags go on from `tag` where that is higher (after a first run); the next
+ * `refuse` launches are refused on the host. */
+psvfwi_status psvfwi_test_resident(psvfwi_plan* plan, int mute, unsigned tag, int refuse);
 
 /* ---- host-side setup (FP64): the inputs the kernels read ---- */
 

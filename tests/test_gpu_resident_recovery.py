@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 # nx, nz, npml, order, fsurf, precision, nt, K: several tiles; strips
 GRIDS = [(101, 77, 8, 4, 1, "fp32", 60, 1.0), (160, 120, 10, 2, 0, "fp64", 45, 1.0), (1900, 700, 20, 4, 0, "fp32", 70, 1.0)]
-FORCE = {"wait": dict(polls=1), "refused": dict(refuse=1)}
+FORCE = {"wait": dict(mute=1), "refused": dict(refuse=1)}
 
 
 def _setup(plan, mode):
@@ -63,6 +63,18 @@ def test_run_is_done_again(grid, mode, how):
     _forward(plan)
     assert all(_same(x, y) for x, y in zip(_adjoint(plan, mode, obs), a))
     assert plan.last_step("adjoint") == (0, False)
+    ref.close()
+    plan.close()
+
+
+def test_wait_runs_out():
+    """Nobody ends the wait but its own count of tries."""
+    print("wait runs out", flush=True)
+    pb, shots, obs = _problem(GRIDS[0], 2, dict(dt=2))
+    ref, plan = (plan_of(pb, "fp32", tz=tz, shots=shots) for tz in (8, None))
+    plan.test_resident(mute=2)
+    assert all(_same(x, y) for x, y in zip(_forward(plan), _forward(ref)))
+    assert plan.last_step("forward") == (8, True)
     ref.close()
     plan.close()
 
