@@ -1,6 +1,8 @@
 """The resident loop's way out: a wait that gives up or a launch that is refused (both forced from
 the host: every kernel still ends by itself) has the run done again with the split step, bit for
 bit, and the exchange's tags may run over."""
+import time
+
 import numpy as np
 import pytest
 
@@ -68,13 +70,19 @@ def test_run_is_done_again(grid, mode, how):
 
 
 def test_wait_runs_out():
-    """Nobody ends the wait but its own count of tries."""
+    """Nobody ends the wait but its own count of tries: long enough for kernels of other processes to
+    leave the GPU, and no more than a few seconds."""
     print("wait runs out", flush=True)
     pb, shots, obs = _problem(GRIDS[0], 2, dict(dt=2))
     ref, plan = (plan_of(pb, "fp32", tz=tz, shots=shots) for tz in (8, None))
+    _forward(plan)
     plan.test_resident(mute=2)
-    assert all(_same(x, y) for x, y in zip(_forward(plan), _forward(ref)))
+    t = time.perf_counter()
+    r = _forward(plan)
+    t = time.perf_counter() - t
+    assert all(_same(x, y) for x, y in zip(r, _forward(ref)))
     assert plan.last_step("forward") == (8, True)
+    assert 1.0 < t < 6.0, t
     ref.close()
     plan.close()
 
