@@ -178,8 +178,6 @@ public:
     // fewest steps of a segment that a resident launch is worth: it loads the whole state and
     // writes it back
     static constexpr int kResidentMin = 8;
-    // ... and from where on the length of a run or segment does not matter
-    static constexpr int kResidentLong = 64;
 
     // ---------------------------------------------------------- plan_setup.cpp
     explicit Plan(const psvfwi_grid_desc& g);
@@ -266,7 +264,7 @@ private:
         bool want = false;      // chosen for a plan with the exact gradient ...
         bool discrete = false;  // ... and its shape has the replay and the reverse steps
         bool uploaded = false;
-        double us = 0, cells = 0;  // what a step takes, and M cells of a launch's tiles
+        double us[3] = {}, cells = 0;  // what a step takes, forward, adjoint, without a gradient; M cells of a launch's tiles
         int rounds = 0;            // launches a step
         int kdiv = 0;           // some CPML K differs from 1
         Partition part;
@@ -320,7 +318,7 @@ private:
     size_t resident_terms() const;
     bool chain_upload() const;
     bool resident_ready();
-    bool resident_for(int steps, bool forward, bool adjoint);
+    bool resident_for(int steps, bool forward, bool adjoint, bool grad = false);
     psvfwi_status resident_points(Tables& t);
     psvfwi_status resident_prepare(std::initializer_list<Tables*> tabs);
     psvfwi_status launch_resident(State<T>& st, Tables& tab, bool fwd_sig, int mode, int kind, int it0, int it1,

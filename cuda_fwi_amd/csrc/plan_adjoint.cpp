@@ -68,7 +68,7 @@ psvfwi_status Plan<T>::adjoint(int flags)
 
     // (checkpoints: the replay of a segment too)
     const bool resident = !(ckpt && ck_used_k_ < kResidentMin) &&
-                          resident_for(ckpt ? std::min(ck_used_k_, ntmax_) : ntmax_, ckpt, true);
+                          resident_for(ckpt ? std::min(ck_used_k_, ntmax_) : ntmax_, ckpt, true, grad);
     if (resident) PSV_TRY(resident_prepare({&adj_tab_}));
     if (resident && ckpt) PSV_TRY(resident_prepare({&fwd_tab_noreceivers_}));
     const int gsize = resident ? res_.conc : group_size();

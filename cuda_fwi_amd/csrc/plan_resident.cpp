@@ -139,14 +139,21 @@ static double strip_move_us(double cells, int esize, int steps)
     return (20.0 + cells * 15 * esize / 4e6) / steps;
 }
 
-// The forward and the adjoint step apart, for runs of few steps.  Split, us a step of `cells` M cells:
-// FP32 forward 11.1 on 0.06, 16.3 on 0.63, 38 on 2.2, 92 on 6.6, adjoint 11.7, 17.8, 45, 122; FP64
-// forward 13.8 on 0.008, 31 on 0.81, 65 on 2.2, adjoint 14.0, 36, 79; compensated FP32 18 on 0.06,
-// 34 on 0.45.
+// The forward and the adjoint step apart.  Split, us a step of `cells` M cells: FP32 forward 11.1 on
+// 0.06, 16.3 on 0.63, 38 on 2.2, 73 on 4.7, 154 on 9.6, 478 on 28, adjoint 11.7, 17.8, 45, 87, 207, 575;
+// FP64 forward 13.8 on 0.008, 31 on 0.81, 65 on 2.2, 154 on 4.7, 370 on 10.6, adjoint 14.0, 36, 79, 206,
+// 438 (above 2 to 7 M the arrays no longer fit in the Infinity Cache); compensated FP32 18 on 0.06, 34 on
+// 0.45.
 static double split_us(double cells, int esize, bool dwords, bool forward)
 {
     if (dwords) return 16.5 + 38.0 * cells;
-    return esize == 4 ? std::max(11.0, 9.0 + (forward ? 12.9 : 17.0) * cells) : 12.0 + (forward ? 23.5 : 31.0) * cells;
+    if (esize == 4) {
+        const double us = forward ? 9.0 + 12.9 * cells + 4.1 * std::max(0.0, cells - 7.0)
+                                  : 9.0 + 17.0 * cells + 4.0 * std::max(0.0, cells - 5.0);
+        return std::max(11.0, us);
+    }
+    const double over = std::max(0.0, cells - 2.2);
+    return forward ? 12.0 + 23.5 * cells + 12.5 * over : 12.0 + 31.0 * cells + 11.0 * over;
 }
 
 // A launch of the resident loop besides its steps, us, where its tiles have `cells` M cells: it
@@ -159,17 +166,20 @@ static double launch_us(double cells, int esize, bool forward)
 }
 
 // Whether the resident loop pays in a run of records or segments of `steps` steps that are run
-// forward, backward or (the replay of a segment) both.  A strip's launches are half a segment long at
-// most.  The line lies where the two sums meet: 8 steps of 3600 x 1200 in FP32, forward, 0.61 ms
-// resident and 0.55 split (12 steps 0.71, 0.81); checkpoints 8 apart there, replay and adjoint of 96
-// steps, 19.4 and 16.2 ms (12 apart 15.1, 16.1); 600 x 300 in FP64, adjoint, 2 steps 0.059 and 0.054
-// (3 steps 0.060, 0.074).
+// forward, backward or (the replay of a segment) both; resident_ready's choice is by the mean of a
+// forward and an adjoint step over a long run.  A strip's launches are half a segment long at most.
+// The line lies where the two sums meet: 8 steps of 3600 x 1200 in FP32, forward, 0.61 ms resident
+// and 0.55 split (12 steps 0.71, 0.81); checkpoints 8 apart there, replay and adjoint of 96 steps,
+// 19.4 and 16.2 ms (12 apart 15.1, 16.1); 600 x 300 in FP64, adjoint, 2 steps 0.059 and 0.054
+// (3 steps 0.060, 0.074); 2000 x 4000 in FP64, where the adjoint step of the largest tiles spills,
+// forward 244 us a step and 298, adjoint 459 and 353.
 template <typename T>
-bool Plan<T>::resident_for(int steps, bool forward, bool adjoint)
+bool Plan<T>::resident_for(int steps, bool forward, bool adjoint, bool grad)
 {
     constexpr bool dwords = std::is_same<T, psv::dfloat>::value;
     constexpr int esize = (int)sizeof(T);
-    const double all = 1e-6 * nslots_ * g_.nzt * g_.nxt;
+    // (the split step's tiles are 64 columns wide: half a column beyond the grid costs what one in it does)
+    const double all = 1e-6 * nslots_ * g_.nzt * (g_.nxt + (double)round_up((size_t)g_.nxt, 64)) / 2;
     double split = 0, least = 0;
     for (bool f : {true, false})
         if (f ? forward : adjoint) {
@@ -177,14 +187,17 @@ bool Plan<T>::resident_for(int steps, bool forward, bool adjoint)
             least += 2.9 + launch_us(all, esize, f) / steps;
         }
     // (no search for a shape where none could pay)
-    if (steps < kResidentLong && least >= split) return false;
-    if (!resident_ready()) return false;
-    if (steps >= kResidentLong) return true;
-    const int most = res_.part.strips.size() > 2 ? std::min(res_.part.steps, (steps + 1) / 2) : steps;
+    if (least >= split || !resident_ready()) return false;
+    // (launches as launch_resident cuts them)
+    int parts = 1;
+    if (res_.part.strips.size() > 2) {
+        parts = (steps + res_.part.steps - 1) / res_.part.steps;
+        parts += steps > 1 ? parts & 1 : 0;
+    }
     double cost = 0;
     for (bool f : {true, false})
         if (f ? forward : adjoint)
-            cost += res_.rounds * (res_.us * (f || esize == 8 ? 1.0 : 1.15) + launch_us(res_.cells, esize, f) / most);
+            cost += res_.rounds * (res_.us[f ? 0 : (grad ? 1 : 2)] + launch_us(res_.cells, esize, f) * parts / steps);
     return cost < split;
 }
 
@@ -233,7 +246,10 @@ bool Plan<T>::resident_ready()
             const double cost = rounds * (shapes[i].us + move);
             if (cost < best) {
                 best = cost;
-                res_.us = shapes[i].us;
+                res_.us[0] = shapes[i].forward;
+                res_.us[1] = shapes[i].adjoint;
+                // without the correlation (2000 x 4000 in FP64, largest tiles: 338 us a step for 459)
+                res_.us[2] = (2 * shapes[i].forward + shapes[i].adjoint) / 3;
                 res_.rounds = rounds;
                 res_.shape = i;
                 res_.conc = conc;
@@ -511,7 +527,7 @@ psvfwi_status Plan<T>::test_resident(int mute, unsigned tag, int refuse)
     template psvfwi_status Plan<T>::test_resident(int, unsigned, int); \
     template Plan<T>::Partition Plan<T>::resident_tiles(const psv::ResShape&, bool, int, int) const; \
     template bool Plan<T>::resident_ready(); \
-    template bool Plan<T>::resident_for(int, bool, bool); \
+    template bool Plan<T>::resident_for(int, bool, bool, bool); \
     template size_t Plan<T>::resident_terms() const; \
     template psvfwi_status Plan<T>::resident_points(Tables&); \
     template psvfwi_status Plan<T>::resident_prepare(std::initializer_list<Tables*>); \

@@ -78,22 +78,27 @@ struct ResidentParams {
     T* g5[5];
 };
 
-// The tile shapes (ResShape) of each type: X(index, waves, rows, rows_edge, us).  12 waves have
-// 168 registers each and 8 have 256, which hold about 9 rows of FP32 and 6 of the 8-byte types.
-#define PSV_RESIDENT_F32(X)                                                                        \
-    X(0, 8, 2, 2, 2.9) X(1, 8, 3, 2, 3.3) X(2, 12, 3, 2, 3.5) X(3, 12, 4, 3, 4.0) X(4, 12, 5, 4, 4.7) \
-    X(5, 12, 6, 4, 5.2) X(6, 12, 7, 5, 6.0) X(7, 12, 8, 5, 7.0) X(8, 12, 9, 5, 7.6)
-#define PSV_RESIDENT_F64(X)                                                                        \
-    X(0, 8, 2, 2, 3.4) X(1, 8, 3, 2, 4.4) X(2, 12, 3, 2, 5.0) X(3, 8, 4, 3, 5.3) X(4, 8, 6, 4, 7.3)   \
-    X(5, 8, 9, 5, 16.5)
-#define PSV_RESIDENT_F32X2(X) X(0, 8, 2, 2, 9.0) X(1, 8, 3, 2, 13.7) X(2, 12, 2, 2, 14.2) X(3, 8, 4, 3, 17.2)
+// The tile shapes (ResShape) of each type: X(index, waves, rows, rows_edge, us, forward, adjoint).
+// 12 waves have 168 registers each and 8 have 256, which hold about 9 rows of FP32 and 6 of the
+// 8-byte types.
+#define PSV_RESIDENT_F32(X)                                                                      \
+    X(0, 8, 2, 2, 2.9, 2.9, 2.9) X(1, 8, 3, 2, 3.3, 3.3, 3.3) X(2, 12, 3, 2, 3.5, 3.5, 3.5)       \
+    X(3, 12, 4, 3, 4.0, 4.0, 4.0) X(4, 12, 5, 4, 4.7, 4.6, 4.8) X(5, 12, 6, 4, 5.2, 5.1, 5.3)     \
+    X(6, 12, 7, 5, 6.0, 5.9, 6.2) X(7, 12, 8, 5, 7.0, 6.8, 7.4) X(8, 12, 9, 5, 7.6, 7.2, 8.8)
+#define PSV_RESIDENT_F64(X)                                                                      \
+    X(0, 8, 2, 2, 3.4, 3.4, 3.4) X(1, 8, 3, 2, 4.4, 4.4, 4.6) X(2, 12, 3, 2, 5.0, 5.0, 5.2)       \
+    X(3, 8, 4, 3, 5.3, 5.3, 5.5) X(4, 8, 6, 4, 7.3, 7.2, 7.4) X(5, 8, 9, 5, 16.5, 11.0, 20.0)
+#define PSV_RESIDENT_F32X2(X)                                                                    \
+    X(0, 8, 2, 2, 9.0, 9.0, 9.0) X(1, 8, 3, 2, 13.7, 13.7, 13.7) X(2, 12, 2, 2, 14.2, 14.2, 14.2) \
+    X(3, 8, 4, 3, 17.2, 17.2, 17.2)
 
 // Tile shapes a launch can take: waves of a workgroup, stacked in z, and rows per wave of
 // the interior and of the edge tiles; us: what a step takes (forward and adjoint mean, order
-// 4, one MI355X, a grid that fills the launch), for the choice among them.
+// 4, one MI355X, a grid that fills the launch), for the choice among them; forward, adjoint: the two
+// apart, for the choice of the split step instead.
 struct ResShape {
     int waves, rows, rows_edge;
-    double us;
+    double us, forward, adjoint;
 };
 
 // The shapes built for a type (sizeof(T) bytes per value), smallest first; returns their

@@ -7,7 +7,7 @@ namespace psv {
 template <>
 const void* resident_kernel_discrete<double>(int order, int mode, int shape, int* threads)
 {
-#define PSV_KERNEL(I, NW, R, RE, US) \
+#define PSV_KERNEL(I, NW, R, RE, US, FWD, ADJ) \
     if (shape == I) { \
         *threads = NW * 64; \
         return kernel_of<double, kReplay, kReverse, NW, R, RE>(order, mode); \

@@ -7,7 +7,7 @@ namespace psv {
 template <>
 int resident_shapes<double>(const ResShape** out)
 {
-#define PSV_SHAPE(I, NW, R, RE, US) {NW, R, RE, US},
+#define PSV_SHAPE(I, NW, R, RE, US, FWD, ADJ) {NW, R, RE, US, FWD, ADJ},
     static const ResShape shapes[] = {PSV_RESIDENT_F64(PSV_SHAPE)};
     *out = shapes;
     return (int)(sizeof shapes / sizeof shapes[0]);
@@ -16,7 +16,7 @@ int resident_shapes<double>(const ResShape** out)
 template <>
 const void* resident_kernel<double>(int order, int mode, int shape, int* threads)
 {
-#define PSV_KERNEL(I, NW, R, RE, US) \
+#define PSV_KERNEL(I, NW, R, RE, US, FWD, ADJ) \
     if (shape == I) { \
         *threads = NW * 64; \
         return kernel_of<double, kForward, kAdjoint, NW, R, RE>(order, mode); \

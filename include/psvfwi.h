@@ -140,9 +140,9 @@ psvfwi_status psvfwi_set_shots(psvfwi_plan* plan, int nshots, const psvfwi_shot_
  * CPML profiles, the grid and the batch allow it and it is expected to be
  * faster, else two launches on tiles of 8 rows.  Random-boundary adjoints
  * (the forward may be resident), snapshot runs, checkpoints less than 8 steps
- * apart, and runs or segments too short to be worth loading the state (one or
- * two steps; on grids of millions of cells up to about 12) take the two
- * launches.  Every choice gives the same results bit for bit. */
+ * apart, runs or segments too short to be worth loading the state (one or two
+ * steps; on grids of millions of cells up to about 12) and gradients on the
+ * largest FP64 grids take the two launches.  Every choice gives the same results bit for bit. */
 psvfwi_status psvfwi_set_tile(psvfwi_plan* plan, int tz);
 
 /* Autotuner: times `steps` forward steps of the current batch with the
