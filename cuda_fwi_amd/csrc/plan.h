@@ -264,7 +264,9 @@ private:
         bool want = false;      // chosen for a plan with the exact gradient ...
         bool discrete = false;  // ... and its shape has the replay and the reverse steps
         bool uploaded = false;
-        double us[3] = {}, cells = 0;  // what a step takes, forward, adjoint, without a gradient; M cells of a launch's tiles
+        // what a step takes: the mean of both kinds; forward, adjoint, adjoint without a gradient
+        double us_mean = 0, us[3] = {};
+        double cells = 0;          // M cells of a launch's tiles
         int rounds = 0;            // launches a step
         int kdiv = 0;           // some CPML K differs from 1
         Partition part;
@@ -318,6 +320,8 @@ private:
     size_t resident_terms() const;
     bool chain_upload() const;
     bool resident_ready();
+    int resident_parts(int steps) const;
+    bool resident_exact(int steps);
     bool resident_for(int steps, bool forward, bool adjoint, bool grad = false);
     psvfwi_status resident_points(Tables& t);
     psvfwi_status resident_prepare(std::initializer_list<Tables*> tabs);

@@ -31,7 +31,7 @@ psvfwi_status Plan<T>::adjoint_discrete()
     }
     // segments of one step: the forward kept every state, no replay
     const bool every = kk == 1;
-    bool resident = kk >= kResidentMin && resident_ready() && res_.discrete;
+    bool resident = kk >= kResidentMin && resident_exact(std::min(kk, ntmax_));
     if (resident) {
         PSV_TRY(resident_prepare({&adj_tab_, &fwd_tab_noreceivers_}));
         PSV_TRY(alloc_state(replay_));

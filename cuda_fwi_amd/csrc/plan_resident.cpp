@@ -162,7 +162,16 @@ static double split_us(double cells, int esize, bool dwords, bool forward)
 // 27 on 0.26, 36 on 0.41, a strip's 51 on 0.85, adjoint 32, 46, 66.
 static double launch_us(double cells, int esize, bool forward)
 {
-    return 20.0 + cells * esize / 4 * (forward ? (esize == 4 ? 17.0 : 16.0) : (esize == 4 ? 36.0 : 25.0));
+    return 20.0 + cells * esize / 4 * (forward ? (esize == 4 ? 17.0 : 20.0) : (esize == 4 ? 36.0 : 25.0));
+}
+
+// Launches of a resident run of `steps` steps, per strip: one, or an even number.
+template <typename T>
+int Plan<T>::resident_parts(int steps) const
+{
+    if (res_.part.strips.size() <= 2) return 1;
+    const int parts = (steps + res_.part.steps - 1) / res_.part.steps;
+    return steps > 1 ? parts + (parts & 1) : parts;
 }
 
 // Whether the resident loop pays in a run of records or segments of `steps` steps that are run
@@ -188,17 +197,29 @@ bool Plan<T>::resident_for(int steps, bool forward, bool adjoint, bool grad)
         }
     // (no search for a shape where none could pay)
     if (least >= split || !resident_ready()) return false;
-    // (launches as launch_resident cuts them)
-    int parts = 1;
-    if (res_.part.strips.size() > 2) {
-        parts = (steps + res_.part.steps - 1) / res_.part.steps;
-        parts += steps > 1 ? parts & 1 : 0;
-    }
+    const int parts = resident_parts(steps);
     double cost = 0;
     for (bool f : {true, false})
         if (f ? forward : adjoint)
             cost += res_.rounds * (res_.us[f ? 0 : (grad ? 1 : 2)] + launch_us(res_.cells, esize, f) * parts / steps);
     return cost < split;
+}
+
+// The same for the exact gradient's segments of `steps` steps, replay and transposed steps.  Resident,
+// the two take about 2.8 forward steps (us a step of a strip: FP32 12 x 9 rows 21.5, FP64 8 x 6 17.5,
+// 8 x 9 46) and their launches 40 us and 62 a M cells of FP32; split, us a step: FP32 28 on 0.06 M cells,
+// 61 on 0.63, 180 on 2.8, 300 on 4.7, 580 on 9.6, FP64 30 on 0.008, 280 on 2.2, 1050 on 8.5, compensated
+// FP32 42 on 0.06.  The line: 2000 x 4000 in FP64, segments of 8 steps 1490 us a step and 1110, of 32
+// 1000 and 1070; 1500 x 6000 in FP32, of 8 710 and 600, of 16 500 and 600.
+template <typename T>
+bool Plan<T>::resident_exact(int steps)
+{
+    if (!resident_ready() || !res_.discrete) return false;
+    constexpr int esize = (int)sizeof(T);
+    const double all = 1e-6 * nslots_ * g_.nzt * g_.nxt;
+    const double split = esize == 4 ? 25.0 + 57.0 * all : (std::is_same<T, psv::dfloat>::value ? 38.0 : 28.0) + 118.0 * all;
+    const double launch = 40.0 + 62.0 * res_.cells * esize / 4;
+    return res_.rounds * (2.8 * res_.us_mean + launch * resident_parts(steps) / steps) < split;
 }
 
 // Whether the plan's runs can take the resident loop, and its shape for the current batch.
@@ -246,6 +267,7 @@ bool Plan<T>::resident_ready()
             const double cost = rounds * (shapes[i].us + move);
             if (cost < best) {
                 best = cost;
+                res_.us_mean = shapes[i].us;
                 res_.us[0] = shapes[i].forward;
                 res_.us[1] = shapes[i].adjoint;
                 // without the correlation (2000 x 4000 in FP64, largest tiles: 338 us a step for 459)
@@ -434,11 +456,7 @@ psvfwi_status Plan<T>::launch_resident(State<T>& st, Tables& tab, bool fwd_sig, 
     // one launch of all steps; strips (one slot at a time): an even number of launches of a few
     // steps each, which ends in the slot's own arrays, each writing the other set of the state
     const int last = nstrip > 1 ? std::min(it1, group_nt()) : it1, n = last - it0;
-    int parts = 1;
-    if (nstrip > 1) {
-        parts = (n + res_.part.steps - 1) / res_.part.steps;
-        parts += n > 1 ? parts & 1 : 0;
-    }
+    const int parts = resident_parts(n);
     hipError_t e = hipSuccess;
     for (int j = 0; j < parts && e == hipSuccess; j++) {
         const bool back = mode == psv::kAdjoint || mode == psv::kReverse;
@@ -528,6 +546,8 @@ psvfwi_status Plan<T>::test_resident(int mute, unsigned tag, int refuse)
     template Plan<T>::Partition Plan<T>::resident_tiles(const psv::ResShape&, bool, int, int) const; \
     template bool Plan<T>::resident_ready(); \
     template bool Plan<T>::resident_for(int, bool, bool, bool); \
+    template bool Plan<T>::resident_exact(int); \
+    template int Plan<T>::resident_parts(int) const; \
     template size_t Plan<T>::resident_terms() const; \
     template psvfwi_status Plan<T>::resident_points(Tables&); \
     template psvfwi_status Plan<T>::resident_prepare(std::initializer_list<Tables*>); \

@@ -180,5 +180,17 @@ def test_large_fp64_adjoint_stays_on_the_split_step():
         plan.adjoint(energy=False)
         out.append(r + list(plan.gradient()))
         assert [plan.last_step(k)[0] for k in ("forward", "adjoint")] == [tz or 0, 8]
-        plan.close()
+        if tz:
+            plan.close()
+    assert all(_same(a, b) for a, b in zip(*out))
+    # its exact gradient: segments of 8 steps 1490 us a step in the loop and 1110 split, of 32 1000 and 1070
+    out = []
+    for k, want in ((8, 8), (32, 0)):
+        plan.set_gradient_mode("discrete", k)
+        plan.forward(energy=False, gradient=True)
+        plan.misfit(obs)
+        plan.adjoint(energy=False)
+        assert plan.last_step("adjoint") == (want, False)
+        out.append(plan.model_gradient())
+    plan.close()
     assert all(_same(a, b) for a, b in zip(*out))
