@@ -259,7 +259,7 @@ private:
     // the resident time loop (plan_resident.cpp): the tiles chosen for a batch of `slots`
     // shots (shape < 0: it does not fit), conc slots per launch
     struct Resident {
-        int slots = 0, shape = -1, conc = 0, cap = 0, waves = 0, rows = 0, rows_edge = 0, gen = 0;
+        int slots = 0, shape = -1, conc = 0, cap = 0, waves = 0, rows = 0, rows_edge = 0, gen = 0, alloc_gen = 0;
         bool failed = false;    // refused or aborted once: the plan keeps to the split step
         bool want = false;      // chosen for a plan with the exact gradient ...
         bool discrete = false;  // ... and its shape has the replay and the reverse steps
@@ -321,6 +321,7 @@ private:
     bool chain_upload() const;
     bool resident_ready();
     int resident_parts(int steps) const;
+    bool resident_alloc();
     bool resident_exact(int steps);
     bool resident_for(int steps, bool forward, bool adjoint, bool grad = false);
     psvfwi_status resident_points(Tables& t);

@@ -202,7 +202,7 @@ bool Plan<T>::resident_for(int steps, bool forward, bool adjoint, bool grad)
     for (bool f : {true, false})
         if (f ? forward : adjoint)
             cost += res_.rounds * (res_.us[f ? 0 : (grad ? 1 : 2)] + launch_us(res_.cells, esize, f) * parts / steps);
-    return cost < split;
+    return cost < split && resident_alloc();
 }
 
 // The same for the exact gradient's segments of `steps` steps, replay and transposed steps.  Resident,
@@ -219,7 +219,7 @@ bool Plan<T>::resident_exact(int steps)
     const double all = 1e-6 * nslots_ * g_.nzt * g_.nxt;
     const double split = esize == 4 ? 25.0 + 57.0 * all : (std::is_same<T, psv::dfloat>::value ? 38.0 : 28.0) + 118.0 * all;
     const double launch = 40.0 + 62.0 * res_.cells * esize / 4;
-    return res_.rounds * (2.8 * res_.us_mean + launch * resident_parts(steps) / steps) < split;
+    return res_.rounds * (2.8 * res_.us_mean + launch * resident_parts(steps) / steps) < split && resident_alloc();
 }
 
 // Whether the plan's runs can take the resident loop, and its shape for the current batch.
@@ -297,40 +297,47 @@ bool Plan<T>::resident_ready()
     res_.cells = 0;
     for (const psv::ResTile& t : res_.part.h) res_.cells += (double)(t.z1 - t.z0) * (t.x1 - t.x0);
     res_.cells *= 1e-6 * (res_.part.strips.size() > 2 ? 1.0 / (res_.part.strips.size() - 1) : res_.conc);
-    // the exchange buffer, the flag, and for strips the other set of a slot's state
-    {
-        res_.xpitch = (int)round_up((size_t)g_.nxt, 8);
-        res_.zpitch = (int)round_up((size_t)g_.nzt, 8);
-        res_.exch_slot = 2 * ((size_t)g_.nzt * res_.xpitch + (size_t)g_.nxt * res_.zpitch) * (2 * sizeof(T) / 4);
-        const size_t need = res_.exch_slot * (size_t)res_.conc;
-        bool ok = true;
-        if (!res_.exch.p || res_.exch.cap < need) {
-            ok = res_.exch.alloc(need) == hipSuccess &&
-                 psv::launch_fill<unsigned long long>(res_.exch.p, need, 0ull, stream_) == hipSuccess;
-            res_.tag = 1;
-        }
-        if (ok && !res_.aborted) {
-            ok = hipHostMalloc(reinterpret_cast<void**>(&res_.aborted), sizeof(int), hipHostMallocMapped) == hipSuccess;
-            if (ok) *res_.aborted = 0;
-        }
-        const bool two = res_.part.strips.size() > 2;
-        for (int k = 0; k < psv::kStateArrays && ok && two; k++) {
-            const size_t n = k < 5 ? fst_ : (g_.npml > 0 ? (k < 9 ? xst_ : zst_) : 0);
-            ok = res_.other[k].alloc(n) == hipSuccess && (n == 0 || psv::launch_fill<T>(res_.other[k].p, n, (T)0, stream_) == hipSuccess);
-        }
-        if (!ok) {
-            (void)hipGetLastError();
-            for (DBuf<T>& b : res_.other) b.release();
-            res_.exch.release();
-            res_.shape = -1;
-            return false;
-        }
-    }
     res_.waves = shapes[res_.shape].waves;
     res_.rows = shapes[res_.shape].rows;
     res_.rows_edge = shapes[res_.shape].rows_edge;
     res_.gen++;
     res_.uploaded = false;
+    return true;
+}
+
+// The memory of the chosen tiles, for a run that takes the loop: the exchange buffer, the flag, and
+// for strips the other set of a slot's state; false (and no loop for this batch) where there is none.
+template <typename T>
+bool Plan<T>::resident_alloc()
+{
+    if (res_.alloc_gen == res_.gen) return true;
+    res_.xpitch = (int)round_up((size_t)g_.nxt, 8);
+    res_.zpitch = (int)round_up((size_t)g_.nzt, 8);
+    res_.exch_slot = 2 * ((size_t)g_.nzt * res_.xpitch + (size_t)g_.nxt * res_.zpitch) * (2 * sizeof(T) / 4);
+    const size_t need = res_.exch_slot * (size_t)res_.conc;
+    bool ok = true;
+    if (!res_.exch.p || res_.exch.cap < need) {
+        ok = res_.exch.alloc(need) == hipSuccess &&
+             psv::launch_fill<unsigned long long>(res_.exch.p, need, 0ull, stream_) == hipSuccess;
+        res_.tag = 1;
+    }
+    if (ok && !res_.aborted) {
+        ok = hipHostMalloc(reinterpret_cast<void**>(&res_.aborted), sizeof(int), hipHostMallocMapped) == hipSuccess;
+        if (ok) *res_.aborted = 0;
+    }
+    const bool two = res_.part.strips.size() > 2;
+    for (int k = 0; k < psv::kStateArrays && ok && two; k++) {
+        const size_t n = k < 5 ? fst_ : (g_.npml > 0 ? (k < 9 ? xst_ : zst_) : 0);
+        ok = res_.other[k].alloc(n) == hipSuccess && (n == 0 || psv::launch_fill<T>(res_.other[k].p, n, (T)0, stream_) == hipSuccess);
+    }
+    if (!ok) {
+        (void)hipGetLastError();
+        for (DBuf<T>& b : res_.other) b.release();
+        res_.exch.release();
+        res_.shape = -1;
+        return false;
+    }
+    res_.alloc_gen = res_.gen;
     return true;
 }
 
@@ -548,6 +555,7 @@ psvfwi_status Plan<T>::test_resident(int mute, unsigned tag, int refuse)
     template bool Plan<T>::resident_for(int, bool, bool, bool); \
     template bool Plan<T>::resident_exact(int); \
     template int Plan<T>::resident_parts(int) const; \
+    template bool Plan<T>::resident_alloc(); \
     template size_t Plan<T>::resident_terms() const; \
     template psvfwi_status Plan<T>::resident_points(Tables&); \
     template psvfwi_status Plan<T>::resident_prepare(std::initializer_list<Tables*>); \

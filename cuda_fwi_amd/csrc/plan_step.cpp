@@ -105,7 +105,7 @@ psvfwi_status Plan<T>::autotune(int steps, int* best)
     // reading and writing of the state is a small part, as in a run
     float res_ms = 1e30f;
     tile_auto_ = true;
-    if (resident_ready()) {
+    if (resident_ready() && resident_alloc()) {
         tz_ = kDefaultTz;
         PSV_TRY(resident_prepare({&adj_tab_, &fwd_tab_noreceivers_}));
         AllSlotsAfter restore{this};
