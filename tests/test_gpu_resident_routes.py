@@ -81,9 +81,10 @@ def test_rounds_of_several_shots(prec):
 
 
 def test_autotuned_tile_serves_the_runs_the_loop_cannot():
-    """On 88 x 88 cells tiles of 4 rows are a quarter to a third faster than any other: the
-    autotuner returns them, and what cannot run resident (snapshots, short checkpoint intervals,
-    the random-boundary adjoint) steps on them."""
+    """On 88 x 88 cells tiles of 8 rows are never the fastest: on the GPU those of 4 are a quarter
+    faster, and where the host's launches set the pace the fused step with one a step is.  The
+    autotuner returns what it measured, and what cannot run resident (snapshots, short checkpoint
+    intervals, the random-boundary adjoint) takes the fastest split tile."""
     print("autotuned tile beside the resident loop", flush=True)
     pb = RC.small_problem(nx=84, nz=84, npml=0, nt=60, fdorder=4, fsurf=0, nrec=6)
     pb.lam, pb.mu, pb.rho = P.random_boundary(pb.lam, pb.mu, pb.rho, 12, 0, seed=5, max_increase=0.3)
@@ -91,18 +92,20 @@ def test_autotuned_tile_serves_the_runs_the_loop_cannot():
     pb.fwi = RC.full_window(pb, dt=2)
     obs = [1e-3 * np.random.default_rng(2).standard_normal((6, pb.nt))]
     plan = plan_of(pb, "fp64")
-    assert plan.autotune(40) == 4
+    best = plan.autotune(40)
+    assert best in (4, 16, -8, -16)
     plan.forward()
     assert plan.last_step("forward") == (0, False)
     plan.set_snapshots(10)
     plan.forward()
-    assert plan.last_step("forward") == (4, False)
+    split = plan.last_step("forward")
+    assert split[0] in ((best,) if best > 0 else (4, 8, 16)) and not split[1]
     plan.set_snapshots(0)
     plan.set_store_mode("checkpoint", 4)
     plan.forward(gradient=True)
     plan.misfit(obs)
     plan.adjoint()
-    assert plan.last_step("forward") == plan.last_step("adjoint") == (4, False)
+    assert plan.last_step("forward") == plan.last_step("adjoint") == split
     g = plan.gradient()
     ref = plan_of(pb, "fp64", tz=8)
     for p in (plan, ref):
@@ -110,7 +113,7 @@ def test_autotuned_tile_serves_the_runs_the_loop_cannot():
         p.forward(gradient=True)
         p.misfit(obs)
         p.adjoint()
-    assert plan.last_step("adjoint") == (4, False)
+    assert plan.last_step("adjoint") == split
     assert all(_same(a, b) for a, b in zip(plan.gradient(), ref.gradient()))
     ref.set_store_mode("full")
     ref.forward(gradient=True)
