@@ -149,16 +149,24 @@ psvfwi_status Plan<T>::autotune(int steps, int* best)
             split_tz = tz_;
         }
     }
-    tz_ = best_tz;
-    PSV_TRY(tune_batch(&best_ms));
-    // the resident loop stays the plan's choice (as set_tile(0) makes it) where it was the
+    // the resident loop stays the plan's choice (as set_tile(0) makes it) where it is the
     // fastest.  The runs that cannot take it (snapshots, the random-boundary adjoint, short
     // segments) then have the fastest split step, not the default: a fused one would swap the
     // loop's state (64 x 64 FP64, forward and adjoint: tiles of 4 rows 2.07 ms, of 8 rows 2.78)
+    bool tuned = false;
     if (res_ms < best_ms) {
-        tile_auto_ = true;
         tz_ = split_tz;
-        if (best_tz != split_tz) PSV_TRY(tune_batch(&split_ms));
+        PSV_TRY(tune_batch(&split_ms));
+        tuned = best_tz == split_tz || split_ms < best_ms;
+        if (tuned) {
+            best_tz = split_tz;
+            best_ms = split_ms;
+        }
+        tile_auto_ = res_ms < best_ms;
+    }
+    if (!tile_auto_ && !tuned) {
+        tz_ = best_tz;
+        PSV_TRY(tune_batch(&best_ms));
     }
     if (best) *best = best_tz;
     // the candidates ran in the plan's own state, store and gradient buffers
